@@ -442,6 +442,7 @@ DEVICE_PRELUDE = r'''
 #define PMX_GLOBAL __attribute__((address_space(1)))
 #define PMX_CONST __attribute__((address_space(4)))
 #define PMX_OPAQUE(x) __asm__ volatile("" : "+v"(x))
+#define PMX_DEVICE_AS 1
 #endif
 __device__ __forceinline__ int pmx_abs(int v) { return v < 0 ? -v : v; }
 __device__ __forceinline__ long long pmx_abs(long long v) { return v < 0 ? -v : v; }

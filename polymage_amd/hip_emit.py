@@ -26,6 +26,8 @@ import re
 from .analysis import PlanError, classify_access, eval_bexpr, unconditional_refs, shift_access, scaled_access
 from .constructs import Reference, Image, Case, Reduction
 from .cprint import Printer, DEVICE_PRELUDE, c_type
+from .box_emit import BOX_PRELUDE, emit_box_kernel
+from .box_plan import BoxPlan
 from .group_plan import GroupPlan
 from .region_ir import REGION_PRELUDE, bound_c
 from .reduction_plan import ReductionPlan, emit_reduction_kernel, ConstPlan, emit_const_kernel
@@ -98,28 +100,25 @@ class _KernelWriter(object):
         self.lines.append('  ' * ind + s)
 
 
-def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
-    """HIP source of one stencil-group kernel."""
-    params = pipe.sorted_parameters()
-    stages = plan.stages
-    # global buffers: out-of-group producers read, live-outs written
+def group_buffers(plan):
+    """(reads, writes, buffers in argument order) of a group kernel:
+    out-of-group producers read, live-outs written."""
     reads = []
-    for s in stages:
+    for s in plan.stages:
         for part in s.parts:
             for r in plan._part_refs(part):
                 f = r.objectRef
                 if not plan.in_group(f) and f not in reads:
                     reads.append(f)
-    writes = [s.func for s in stages if s.liveout]
-    buffers = sorted(reads, key=lambda f: f.name) + sorted(writes, key=lambda f: f.name)
-    index_t = 'long long' if plan.opts.get('index64') else 'int'
+    writes = [s.func for s in plan.stages if s.liveout]
+    return reads, writes, sorted(reads, key=lambda f: f.name) + sorted(writes, key=lambda f: f.name)
 
-    base_pr = Printer({}, None, mode)
-    L = []
-    w = lambda s, ind=1: L.append('  ' * ind + s)
 
-    # tile indices
-    total = plan.total_tiles
+def tile_lines(plan, base_pr, xcd):
+    """Statements decoding the workgroup's tile indices t<d> (and the tile
+    counts n<d>) from pmx_tile."""
+    out = []
+    w = out.append
     w('int pmx_b = pmx_tile;')
     a = plan.anchor
     grid = plan.grid_dims
@@ -150,6 +149,54 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
             w('if (t%d >= n%d) return;' % (d, d))
         else:
             w('const int t%d = pmx_b %% n%d; pmx_b /= n%d;' % (d, d, d))
+    return out
+
+
+def stride_lines(buffers, base_pr, index_t):
+    """Extents E_, lower bounds LB_ and strides S_ of the global arrays."""
+    out = []
+    for f in buffers:
+        nd = len(f.domain)
+        for d in range(nd):
+            out.append('const %s E_%s_%d = %s;' % (index_t, f.name, d, _extent_c(f, d, base_pr)))
+            out.append('const int LB_%s_%d = %s;' % (f.name, d, base_pr.expr(f.domain[d].lowerBound)))
+        for d in range(nd - 1):
+            out.append('const %s S_%s_%d = %s;' % (index_t, f.name, d, ' * '.join(
+                'E_%s_%d' % (f.name, j) for j in range(d + 1, nd))))
+    return out
+
+
+def grid_exprs(plan, base_pr, roll):
+    """C expressions (host, parameters in scope) of a group kernel's number
+    of workgroups and of tiles."""
+    a = plan.anchor
+    grid = plan.grid_dims
+    roll_d = next((d for (d, T) in grid if T > 1), None)
+    tiles_c = ' * '.join('((%s + %d) / %d)' % (_extent_c(a.func, d, base_pr), T - 1, T)
+                         for (d, T) in grid) or '1'
+    grid_c = ' * '.join(('((((%s + %d) / %d) + %d) / %d)' % (_extent_c(a.func, d, base_pr), T - 1, T,
+                                                              roll - 1, roll))
+                        if d == roll_d else
+                        '((%s + %d) / %d)' % (_extent_c(a.func, d, base_pr), T - 1, T)
+                        for (d, T) in grid) or '1'
+    return grid_c, tiles_c
+
+
+def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
+    """HIP source of one stencil-group kernel."""
+    params = pipe.sorted_parameters()
+    stages = plan.stages
+    reads, writes, buffers = group_buffers(plan)
+    index_t = 'long long' if plan.opts.get('index64') else 'int'
+
+    base_pr = Printer({}, None, mode)
+    L = []
+    w = lambda s, ind=1: L.append('  ' * ind + s)
+
+    a = plan.anchor
+    grid = plan.grid_dims
+    for l in tile_lines(plan, base_pr, xcd):
+        w(l)
 
     # extra prologue values: part boxes of every stage
     ir = plan.ir
@@ -164,16 +211,8 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
         w(l)
     R = lambda i: 'r%d' % i
 
-    # global strides
-    gfun = buffers
-    for f in gfun:
-        nd = len(f.domain)
-        for d in range(nd):
-            w('const %s E_%s_%d = %s;' % (index_t, f.name, d, _extent_c(f, d, base_pr)))
-            w('const int LB_%s_%d = %s;' % (f.name, d, base_pr.expr(f.domain[d].lowerBound)))
-        for d in range(nd - 1):
-            w('const %s S_%s_%d = %s;' % (index_t, f.name, d, ' * '.join(
-                'E_%s_%d' % (f.name, j) for j in range(d + 1, nd))))
+    for l in stride_lines(buffers, base_pr, index_t):
+        w(l)
 
     def gindex(f, idx_strs):
         e = None
@@ -870,14 +909,8 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
         w('}', 2)
         w('}', 2)
         w('}')
-    roll = max(1, int(plan.opts.get('roll', 1))) if roll_d is not None else 1
-    tiles_c = ' * '.join('((%s + %d) / %d)' % (_extent_c(a.func, d, base_pr), T - 1, T)
-                         for (d, T) in grid) or '1'
-    grid_c = ' * '.join(('((((%s + %d) / %d) + %d) / %d)' % (_extent_c(a.func, d, base_pr), T - 1, T,
-                                                              roll - 1, roll))
-                        if d == roll_d else
-                        '((%s + %d) / %d)' % (_extent_c(a.func, d, base_pr), T - 1, T)
-                        for (d, T) in grid) or '1'
+    roll = max(1, int(plan.opts.get('roll', 1))) if any(T > 1 for (d, T) in grid) else 1
+    grid_c, tiles_c = grid_exprs(plan, base_pr, roll)
     info = KernelInfo(kname, 'group', buffers, grid_c, threads, plan.lds_bytes, plan, reads, writes)
     info.tiles_c = tiles_c
     return wrap_kernel(kname, params, buffers, writes, threads, plan.lds_bytes, L, roll=roll), info
@@ -1266,6 +1299,18 @@ def plan_pipeline(pipe):
     return plans
 
 
+def _emit_group(pipe, plan, kname, threads, mode, xcd):
+    """The box kernel of a group that has constant boxes, else the general
+    kernel."""
+    box = BoxPlan.of(plan)
+    if box is not None:
+        try:
+            return emit_box_kernel(pipe, box, kname, threads, mode, xcd)
+        except PlanError:
+            pass
+    return emit_group_kernel(pipe, plan, kname, threads, mode, xcd)
+
+
 def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
     mode = pipe.literal_mode
     opts = pipe.gpu_options
@@ -1273,7 +1318,7 @@ def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
     xcd = bool(opts.get('xcd_swizzle', True))
     plans = plan_pipeline(pipe)
     srcs = ['// generated by polymage_amd for pipeline %s' % pipe.name,
-            DEVICE_PRELUDE, REGION_PRELUDE,
+            DEVICE_PRELUDE, REGION_PRELUDE, BOX_PRELUDE,
             'extern "C" __global__ void pmx_zero_u64(unsigned long long* p, const int n) {\n'
             '  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);\n'
             '  if (i < n) p[i] = 0ULL;\n}\n']
@@ -1282,7 +1327,7 @@ def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
     for i, plan in enumerate(plans):
         kname = 'pmx_%s_g%d' % (pipe.name, i)
         if isinstance(plan, GroupPlan):
-            src, info = emit_group_kernel(pipe, plan, kname, threads, mode, xcd)
+            src, info = _emit_group(pipe, plan, kname, threads, mode, xcd)
         elif isinstance(plan, ReductionPlan):
             for src, info in emit_reduction_kernel(pipe, plan, kname, mode):
                 srcs.append(src)
