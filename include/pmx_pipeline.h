@@ -58,8 +58,8 @@ extern "C" {
  *       return -12 before anything is launched.  Every such call on a GPU
  *       shares that GPU's scratch: calls that overlap on one GPU race.
  *
- * Batched frames (no reference counterpart; the persistent work-queue
- * path for many small or uneven frames):
+ * Batched frames (no reference counterpart; one launch per kernel
+ * for many small or uneven frames):
  *
  *   int pipeline_<name>_batch_create(int n, const P* P_arr...,
  *                                    void* const* I_arr..., void* const* O_arr...,
@@ -67,7 +67,7 @@ extern "C" {
  *       n frames; per-frame parameters and device pointers; validates every
  *       frame and builds the frame tables on the device.
  *   int pipeline_<name>_batch_run(void* handle, void* stream);
- *       one persistent launch per group over all frames' tiles.
+ *       one launch per kernel over all frames' tiles (a workgroup each).
  *   int pipeline_<name>_batch_run_graph(void* handle, void* stream);
  *       the same launches captured once into a hipGraph, replayed.
  *   int pipeline_<name>_batch_run_frames(void* handle, void* stream);

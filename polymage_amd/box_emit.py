@@ -25,7 +25,7 @@ from .region_ir import bound_c
 
 # device helpers of box kernels: a pointer moved by a byte offset, and
 # stores of short vectors at element alignment (gfx950's global memory takes
-# them unaligned).  The overloads keep the address space of the persistent
+# them unaligned).  The overloads keep the address space of the batch
 # kernels' pointers.
 BOX_PRELUDE = r'''
 template <typename T, int N> struct pmx_vec {

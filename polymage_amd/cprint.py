@@ -441,7 +441,6 @@ DEVICE_PRELUDE = r'''
 #ifndef PMX_GLOBAL
 #define PMX_GLOBAL __attribute__((address_space(1)))
 #define PMX_CONST __attribute__((address_space(4)))
-#define PMX_OPAQUE(x) __asm__ volatile("" : "+v"(x))
 #define PMX_DEVICE_AS 1
 #endif
 __device__ __forceinline__ int pmx_abs(int v) { return v < 0 ? -v : v; }
@@ -478,6 +477,28 @@ __device__ __forceinline__ double pmx_fmad(double a, double b, double c) { retur
 __device__ __forceinline__ double pmx_divc(double n, double r, double d) {
   const double q = n * r;
   return __builtin_fma(__builtin_fma(-q, d, n), r, q);
+}
+// last frame whose first work item (ascending, in memory) is <= t
+__device__ __forceinline__ int pmx_find_frame(const long long* first, const int n, const long long t) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) { const int mid = (lo + hi + 1) >> 1; if (first[mid] <= t) lo = mid; else hi = mid - 1; }
+  return lo;
+}
+// the same for wavefronts of 64 active lanes, 64 frames per step, one a lane
+// (a search by halves is a chain of six dependent loads for 48 frames)
+__device__ __forceinline__ int pmx_find_frame64(const long long* first, const int n, const long long t) {
+#ifdef PMX_DEVICE_AS
+  int c = 0;
+  for (int b = 0; b < n; b += 64) {
+    const int i = b + (int)(threadIdx.x & 63u);
+    const int k = __popcll(__ballot(i < n && first[i < n ? i : 0] <= t));
+    c += k;
+    if (k < 64) break;
+  }
+  return __builtin_amdgcn_readfirstlane(c - 1);
+#else
+  return pmx_find_frame(first, n, t);
+#endif
 }
 #ifndef PMX_LD4
 #define PMX_LD4 1

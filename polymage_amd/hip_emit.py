@@ -1174,12 +1174,17 @@ def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines, 
     """The kernel body as a device function plus two entry points:
 
     ``<k>``       one workgroup per tile (grid = number of tiles);
-    ``<k>_batch`` persistent: a fixed set of workgroups pulls (frame, tile)
-                  work items from 8 atomic queues (one per XCD) until all
-                  are empty; frames are described by ``<k>_frame`` records
+    ``<k>_batch`` one workgroup per (frame, tile) work item over all frames
+                  of a batch; frames are described by ``<k>_frame`` records
                   (buffers, first global work item, parameters).
-    Every workgroup of the persistent form leaves the loop once all 8
-    counters have passed their queue's end, so the grid always drains."""
+
+    The batch form used to keep a resident grid that pulled items from
+    queues with atomics.  An item's fetch then sat in front of its loads
+    (the memory counter retires in order), two more barriers closed every
+    item, and a workgroup's items ran one after another; the hardware's own
+    dispatch of one workgroup per item overlaps them (48 camera frames,
+    88 k items of 32 x 32: 1275 us with the queues, 881 us so).  ``first`` is the launch's first item: a batch of more
+    items than one grid holds is launched in pieces."""
     decls, names, fields = kernel_args(params, buffers, writes)
     lds = max(16, lds_bytes)
     tail = ['const int pmx_tile', 'const int pmx_remap', 'const int pmx_rk', 'const int pmx_rr',
@@ -1191,13 +1196,11 @@ def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines, 
          prologue, '  const int pmx_tx = (int)threadIdx.x; (void)pmx_tx;']
     L += body_lines
     L.append('}')
-    # persistent form: the same body over pointers read from frame records.
+    # batch form: the same body over pointers read from frame records.
     # Buffers the kernel writes are global-address-space pointers (global,
     # not flat, stores); buffers it only reads are constant-address-space
     # pointers (they do not change during the launch, so reads at uniform
-    # addresses become scalar loads).  The thread index is opaque to the
-    # optimiser, so per-thread index arithmetic is recomputed for every work
-    # item instead of being hoisted out of the work loop into registers.
+    # addresses become scalar loads).
     ptypes = {'pmx_err': 'int'}
     for f in buffers:
         ptypes['G_' + f.name] = ('' if f in writes else 'const ') + c_type(f.typ)
@@ -1208,7 +1211,7 @@ def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines, 
     fargs = ['(%s %s*)f.%s' % (ptypes[n], aspace[n], n) if n in ptypes else 'f.' + n
              for n in names]
     L += ['__device__ __forceinline__ void %s_bbody(%s) {' % (kname, ', '.join(bdecls + tail)),
-          prologue, '  int pmx_tx = (int)threadIdx.x; PMX_OPAQUE(pmx_tx); (void)pmx_tx;']
+          prologue, '  const int pmx_tx = (int)threadIdx.x; (void)pmx_tx;']
     L += body_lines
     L.append('}')
     L.append('extern "C" __global__ __launch_bounds__(%d) void %s(%s) {' % (
@@ -1226,58 +1229,27 @@ def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines, 
     L.append('}')
     L.append('struct %s_frame { %s };' % (kname, ' '.join(fields)))
     L.append('extern "C" __global__ __launch_bounds__(%d) void %s_batch(const %s_frame* __restrict__ F, '
-             'const int nframes, unsigned long long* __restrict__ counter, const long long total) {'
+             'const int nframes, const long long first, const long long total) {'
              % (threads, kname, kname))
     L.append('  __shared__ __align__(16) unsigned char pmx_lds[%d];' % lds)
-    L.append('  __shared__ long long pmx_work;')
     L.append('  // frame records do not change during the launch: read through the')
     L.append('  // constant address space they are scalar loads')
     L.append('  const %s_frame PMX_CONST* __restrict__ Fc = (const %s_frame PMX_CONST*)F;' % (kname, kname))
-    L.append('  // 8 queues, one per XCD (workgroups are dealt round-robin to the')
-    L.append('  // XCDs): queue q holds the contiguous items [total*q/8, total*(q+1)/8),')
-    L.append('  // so neighbouring tiles share an L2; an empty home queue sends the')
-    L.append('  // workgroup on to the next ones until all 8 are empty.  The next')
-    L.append('  // item is fetched while the current one is processed.')
-    L.append('  const int home = (int)(blockIdx.x & 7);')
-    L.append('  int q = 0;')
-    L.append('  auto pmx_fetch = [&]() -> long long {')
-    L.append('    while (q < 8) {')
-    L.append('      const int qq = (home + q) & 7;')
-    L.append('      const long long lo = total * qq / 8, hi = total * (qq + 1) / 8;')
-    L.append('      const long long k = (long long)atomicAdd(&counter[qq], 1ULL);')
-    L.append('      if (lo + k < hi) return lo + k;')
-    L.append('      ++q;')
-    L.append('    }')
-    L.append('    return -1;')
-    L.append('  };')
-    L.append('  if (threadIdx.x == 0) pmx_work = pmx_fetch();')
-    L.append('  __syncthreads();')
-    L.append('  for (;;) {')
-    L.append('    // the work item and its frame are the same for the whole workgroup:')
-    L.append('    // readfirstlane makes that visible, so the frame record (copied')
-    L.append('    // word by word) and all per-tile index arithmetic stay in scalar')
-    L.append('    // registers')
-    L.append('    const long long tw = pmx_work;')
-    L.append('    const long long t = (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane('
-             '(int)(tw >> 32)) << 32) | (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)tw));')
-    L.append('    if (t < 0) break;')
-    L.append('    long long nxt = -1;')
-    L.append('    if (threadIdx.x == 0) nxt = pmx_fetch();')
-    L.append('    // the frame holding work item t: last frame whose first item is <= t')
-    L.append('    int lo = 0, hi = nframes - 1;')
-    L.append('    while (lo < hi) { const int mid = (lo + hi + 1) >> 1; if (Fc[mid].pmx_tile0 <= t) lo = mid; else hi = mid - 1; }')
-    L.append('    lo = __builtin_amdgcn_readfirstlane(lo);')
-    L.append('    %s_frame f;' % kname)
-    L.append('    { int w[sizeof(f) / 4]; __builtin_memcpy(w, (const void*)&Fc[lo], sizeof(f));')
-    L.append('      for (int i = 0; i < (int)(sizeof(f) / 4); ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);')
-    L.append('      __builtin_memcpy(&f, w, sizeof(f)); }')
-    L.append('    %s_bbody(%s);' % (kname, ', '.join(fargs +
-                                                   ['(int)(t - f.pmx_tile0)', '0', '0', '1',
-                                                    'pmx_lds'])))
-    L.append('    __syncthreads();')
-    L.append('    if (threadIdx.x == 0) pmx_work = nxt;')
-    L.append('    __syncthreads();')
-    L.append('  }')
+    L.append('  // workgroups are dealt round-robin to the 8 XCDs: give each XCD a')
+    L.append('  // contiguous eighth of the items, so neighbouring tiles share an L2')
+    L.append('  const long long per = (total + 7) / 8;')
+    L.append('  const long long t = first + (long long)(blockIdx.x & 7) * per + (long long)(blockIdx.x >> 3);')
+    L.append('  if ((long long)(blockIdx.x >> 3) >= per || t >= first + total) return;')
+    L.append('  // the frame holding item t, and its record (copied word by word:')
+    L.append('  // readfirstlane keeps it and all per-tile index arithmetic in scalar')
+    L.append('  // registers)')
+    L.append('  const int lo = __builtin_amdgcn_readfirstlane(pmx_find_frame%s((const long long*)(F + nframes), nframes, t));'
+             % ('64' if threads % 64 == 0 else ''))
+    L.append('  %s_frame f;' % kname)
+    L.append('  { int w[sizeof(f) / 4]; __builtin_memcpy(w, (const void*)&Fc[lo], sizeof(f));')
+    L.append('    for (int i = 0; i < (int)(sizeof(f) / 4); ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);')
+    L.append('    __builtin_memcpy(&f, w, sizeof(f)); }')
+    L.append('  %s_bbody(%s);' % (kname, ', '.join(fargs + ['(int)(t - f.pmx_tile0)', '0', '0', '1', 'pmx_lds'])))
     L.append('}')
     return '\n'.join(L) + '\n'
 
@@ -1318,10 +1290,7 @@ def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
     xcd = bool(opts.get('xcd_swizzle', True))
     plans = plan_pipeline(pipe)
     srcs = ['// generated by polymage_amd for pipeline %s' % pipe.name,
-            DEVICE_PRELUDE, REGION_PRELUDE, BOX_PRELUDE,
-            'extern "C" __global__ void pmx_zero_u64(unsigned long long* p, const int n) {\n'
-            '  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);\n'
-            '  if (i < n) p[i] = 0ULL;\n}\n']
+            DEVICE_PRELUDE, REGION_PRELUDE, BOX_PRELUDE]
     kernels = []
     host_consts = []
     for i, plan in enumerate(plans):

@@ -114,7 +114,6 @@ def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_
     w('static void* pmx_mod[64];')
     w('static void* pmx_fn[64][%d];' % max(1, nk))
     w('static void* pmx_fn_batch[64][%d];' % max(1, nk))
-    w('static void* pmx_zero_fn[64];')
     w('static int pmx_load(int dev) {')
     w('  if (dev < 0 || dev >= 64) { pmx_set_error("device index"); return -1; }')
     w('  if (pmx_mod[dev]) return 0;')
@@ -123,7 +122,6 @@ def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_
     w('  for (int k = 0; k < %d; ++k) { rc = pmx_module_function(m, pmx_kernel_names[k], &pmx_fn[dev][k]); if (rc) return rc; }' % nk)
     w('  for (int k = 0; k < %d; ++k) { char nm[256]; snprintf(nm, sizeof nm, "%%s_batch", pmx_kernel_names[k]); '
       'rc = pmx_module_function(m, nm, &pmx_fn_batch[dev][k]); if (rc) return rc; }' % nk)
-    w('  rc = pmx_module_function(m, "pmx_zero_u64", &pmx_zero_fn[dev]); if (rc) return rc;')
     w('  pmx_mod[dev] = m;')
     w('  return 0;')
     w('}')
@@ -302,8 +300,8 @@ def _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None):
         per-frame input pointer arrays..., per-frame output pointer arrays...,
         &handle): plans every kernel's work items over all frames, allocates
         per-frame intermediates, uploads the frame records.
-    pipeline_<name>_batch_run(handle, stream): one persistent work-queue
-        launch per kernel for all frames.
+    pipeline_<name>_batch_run(handle, stream): one launch per kernel over
+        the work items (frame, tile) of all frames.
     pipeline_<name>_batch_run_graph(handle, stream): the same sequence
         captured once in a hipGraph and replayed.
     pipeline_<name>_batch_run_frames(handle, stream): the per-frame plain
@@ -323,9 +321,8 @@ def _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None):
     w('  int n = 0; int dev = 0;')
     w('  void* frames[%d] = {};' % max(1, nk))
     w('  long long total[%d] = {};' % max(1, nk))
-    w('  void* counters = nullptr; void* graph = nullptr;')
+    w('  void* graph = nullptr;')
     w('  std::vector<void*> owned;  // per-frame intermediates of this handle')
-    w('  long long grid[%d] = {};' % max(1, nk))
     for p in params:
         w('  std::vector<%s> p_%s;' % (c_type(p.typ), p.name))
     for f in inputs + outputs:
@@ -336,7 +333,6 @@ def _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None):
     w('  if (!B) return 0;')
     w('  if (B->graph) pmx_graph_destroy(B->graph);')
     w('  for (int k = 0; k < %d; ++k) if (B->frames[k]) pmx_free(B->frames[k]);' % max(1, nk))
-    w('  if (B->counters) pmx_free(B->counters);')
     w('  for (void* p : B->owned) pmx_free(p);')
     w('  delete B;')
     w('  return 0;')
@@ -395,18 +391,17 @@ def _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None):
     for ki, k in enumerate(kernels):
         w('  { long long acc = 0; for (int i = 0; i < n; ++i) { long long c = rec_%s[i].pmx_tile0; '
           'rec_%s[i].pmx_tile0 = acc; acc += c; } B->total[%d] = acc; }' % (k.name, k.name, ki))
-        w('  rc = pmx_malloc(&B->frames[%d], sizeof(%s_frame) * (size_t)n); if (rc) { pmx_batch_%s_free(B); return rc; }'
+        # the frame records, then every frame's first work item once more,
+        # side by side (the kernel finds an item's frame in them)
+        w('  std::vector<long long> first_%s((size_t)n); for (int i = 0; i < n; ++i) first_%s[i] = rec_%s[i].pmx_tile0;'
+          % (k.name, k.name, k.name))
+        w('  rc = pmx_malloc(&B->frames[%d], (sizeof(%s_frame) + sizeof(long long)) * (size_t)n); if (rc) { pmx_batch_%s_free(B); return rc; }'
           % (ki, k.name, name))
         w('  rc = pmx_memcpy_h2d(B->frames[%d], rec_%s.data(), sizeof(%s_frame) * (size_t)n, nullptr); '
           'if (rc) { pmx_batch_%s_free(B); return rc; }' % (ki, k.name, k.name, name))
-    # persistent grids: as many workgroups as stay resident on the device
-    w('  { int cus = 0; rc = pmx_device_cus(B->dev, &cus); if (rc) { pmx_batch_%s_free(B); return rc; }' % name)
-    for ki, k in enumerate(kernels):
-        w('    { int occ = 0; rc = pmx_occupancy(pmx_fn_batch[B->dev][%d], %d, 0, &occ); '
-          'if (rc) { pmx_batch_%s_free(B); return rc; } if (occ < 1) occ = 1; B->grid[%d] = (long long)occ * cus; }'
-          % (ki, k.threads, name, ki))
-    w('  }')
-    w('  rc = pmx_malloc(&B->counters, 64 * %d); if (rc) { pmx_batch_%s_free(B); return rc; }' % (max(1, nk), name))
+        w('  rc = pmx_memcpy_h2d((%s_frame*)B->frames[%d] + n, first_%s.data(), sizeof(long long) * (size_t)n, nullptr); '
+          'if (rc) { pmx_batch_%s_free(B); return rc; }' % (k.name, ki, k.name, name))
+    # (the uploads above read the vectors until this synchronisation)
     w('  rc = pmx_stream_sync(nullptr); if (rc) { pmx_batch_%s_free(B); return rc; }' % name)
     w('  *handle = (void*)B;')
     w('  return 0;')
@@ -414,14 +409,14 @@ def _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None):
     w('extern "C" int pipeline_%s_batch_run(void* handle, void* stream) {' % name)
     w('  pmx_batch_%s* B = (pmx_batch_%s*)handle;' % (name, name))
     w('  int rc = pmx_load(B->dev); if (rc) return rc;')
-    w('  { void* c = B->counters; int nc = %d; void* args[] = {&c, &nc};' % (8 * max(1, nk)))
-    w('    rc = pmx_launch(pmx_zero_fn[B->dev], 1, 1, 1, 64, 1, 1, 0, stream, args); if (rc) return rc; }')
     for ki, k in enumerate(kernels):
-        w('  { void* f = B->frames[%d]; int n = B->n; unsigned long long* c = (unsigned long long*)B->counters + %d; '
-          'long long t = B->total[%d];' % (ki, 8 * ki, ki))
-        w('    void* args[] = {&f, &n, &c, &t};')
-        w('    long long g = t < B->grid[%d] ? t : B->grid[%d];' % (ki, ki))
-        w('    if (g > 0) { rc = pmx_launch(pmx_fn_batch[B->dev][%d], (unsigned)g, 1, 1, %d, 1, 1, 0, stream, args); if (rc) return rc; } }'
+        # a grid holds fewer than 2^32 threads: larger batches go in pieces
+        most = ((1 << 31) // k.threads) // 8 * 8
+        w('  for (long long first = 0; first < B->total[%d]; first += %dLL) {' % (ki, most))
+        w('    void* f = B->frames[%d]; int n = B->n; long long c = B->total[%d] - first < %dLL ? B->total[%d] - first : %dLL;'
+          % (ki, ki, most, ki, most))
+        w('    void* args[] = {&f, &n, &first, &c};')
+        w('    rc = pmx_launch(pmx_fn_batch[B->dev][%d], (unsigned)((c + 7) / 8 * 8), 1, 1, %d, 1, 1, 0, stream, args); if (rc) return rc; }'
           % (ki, k.threads))
     w('  return 0;')
     w('}')

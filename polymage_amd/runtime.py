@@ -128,7 +128,7 @@ class BuiltPipeline(object):
             args.append(ctypes.c_void_p(a.ctypes.data))
         check(self.fn_host_rc(*args), 'pipeline_%s' % self.name)
 
-    # -- batches of frames (persistent work-queue launches) ----------------
+    # -- batches of frames (one launch per kernel over all frames) ----------------
     def batch_create(self, frames):
         """frames: list of dicts like run_dev's ``values`` (device
         pointers).  Returns an opaque handle for batch_run*."""

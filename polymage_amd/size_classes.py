@@ -5,7 +5,7 @@ A batch of frames (the camera pipeline's 48 frames of 384x512 to
 The autotuner searches each class's schedule on a representative frame
 size (``autotune --size-classes campipe:3``) and records it in
 ``tuned.json`` under the application's ``classes``.  ``ClassedBatch`` then
-runs the frames of each class through a persistent work-queue launch of
+runs the frames of each class through one launch over the work items of
 that class's own compiled pipeline (or the class's captured graph), one
 launch per class on one stream, so every class uses the tiles tuned for
 frames of its size.

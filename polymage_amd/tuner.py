@@ -533,7 +533,7 @@ def time_candidates(workload, compiled, runs=9, db=None, app=None, verbose=False
 
 
 def time_batch(bp, workload, frames, frame_input='img', runs=5, warmup=1, reps=3):
-    """Milliseconds per persistent work-queue launch of ``bp`` over a batch
+    """Milliseconds per batched launch of ``bp`` over a batch
     of frames (``frames``: input arrays of the workload's ``frame_input``,
     of any sizes; the workload function gives every other value and the
     output shape at each frame's size), device-resident; median of ``reps``

@@ -129,3 +129,53 @@ def test_box_kernels_bitexact(gpu, app, R, C, tiles, dt):
     print("case box", app, R, C, tiles, dt, flush=True)
     out, pipe, vals, shape = _case(app, R, C, tiles, dt)
     _check(out, gpu_build(pipe).run_host, vals, shape)
+
+
+def _small_frames(n):
+    """n Harris frames of uneven sizes (some of one tile) and their outputs."""
+    from polymage_amd.apps.harris import harris_pipe
+    pd = {}
+    out = harris_pipe(pd)
+    pipe = build(out, pd, {'R': 62, 'C': 94}, 'harris', [16, 32])
+    orc = cemit.build([out], 'box_harris')
+    g = np.random.default_rng(n)
+    recs, refs = [], []
+    for k in range(n):
+        R, C = 5 + (7 * k) % 40, 6 + (11 * k) % 60
+        vals = {'R': R, 'C': C, 'img': g.random((R + 2, C + 2)).astype(np.float32)}
+        o = np.full((R + 2, C + 2), -7.0, np.float32)
+        orc(dict(vals, harris=o))
+        refs.append(o)
+        recs.append(dict(vals, harris=np.full_like(o, -7.0)))
+    return pipe, recs, refs
+
+
+def test_batch_of_many_frames_on_the_emulator():
+    import kernel_emu
+    pipe, recs, refs = _small_frames(5)
+    kernel_emu.build(pipe).run_batch(recs, 'persistent')
+    assert all(bits_equal(rec['harris'], r) for rec, r in zip(recs, refs))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 130])
+def test_batch_of_many_frames(gpu, n):
+    """A work item's frame is found 64 frames a step."""
+    if emulating():
+        pytest.skip("device tensors are not emulated")
+    import torch
+    print("case batch frames", n, flush=True)
+    pipe, recs, refs = _small_frames(n)
+    bp = gpu_build(pipe)
+    dev = [dict(rec, img=torch.from_numpy(rec['img']).cuda(), harris=torch.from_numpy(rec['harris']).cuda())
+           for rec in recs]
+    h = bp.batch_create(dev)
+    try:
+        for mode in ('persistent', 'graph', 'graph'):
+            for d in dev:
+                d['harris'].fill_(-7.0)
+            bp.batch_run(h, torch.cuda.current_stream().cuda_stream, mode)
+            torch.cuda.synchronize()
+            assert all(bits_equal(d['harris'].cpu().numpy(), r) for d, r in zip(dev, refs))
+    finally:
+        bp.batch_destroy(h)
