@@ -442,6 +442,11 @@ DEVICE_PRELUDE = r'''
 #define PMX_GLOBAL __attribute__((address_space(1)))
 #define PMX_CONST __attribute__((address_space(4)))
 #define PMX_DEVICE_AS 1
+#define PMX_SCHED_BARRIER __builtin_amdgcn_sched_barrier(0)
+#define PMX_ALL(x) __all(x)
+#else
+#define PMX_SCHED_BARRIER
+#define PMX_ALL(x) (x)
 #endif
 __device__ __forceinline__ int pmx_abs(int v) { return v < 0 ? -v : v; }
 __device__ __forceinline__ long long pmx_abs(long long v) { return v < 0 ? -v : v; }
