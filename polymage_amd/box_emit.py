@@ -245,10 +245,22 @@ class _Item(object):
         B = self.B
         maps = [arg_map(a, t.func.variables) for a in ref.arguments]
         nd = len(maps)
-        static = all(m.kind != '*' for m in maps)
+        # (edge tiles clamp every index of a data-dependent read: its other
+        # indices may lie outside the array for points that do not count)
+        static = not B.edge or all(m.kind != '*' for m in maps)
         xs = []
+        dyn = []
         if static:
-            for m in maps:
+            for i, m in enumerate(maps):
+                if m.kind == '*':
+                    # clamped; its offset is added to the item's
+                    q = 'pmx_clampi(%s, LB_%s_%d, LB_%s_%d + (int)E_%s_%d - 1)' % (
+                        pr.expr(ref.arguments[i], pro), f.name, i, f.name, i, f.name, i)
+                    dyn.append('(unsigned)(%s - LB_%s_%d) * %s' % (
+                        q, f.name, i, '(unsigned)(S_%s_%d * %d)' % (f.name, i, f.typ.nbytes())
+                        if i < nd - 1 else '%du' % f.typ.nbytes()))
+                    xs.append(None)
+                    continue
                 if m.kind == 'const':
                     xs.append((m.value, {}, Span(None, 0, m.value, m.value)))
                     continue
@@ -260,6 +272,8 @@ class _Item(object):
                 xs.append((x[0], x[1], Span(sp.d, int(m.slope * sp.A), m.f(sp.lo), m.f(sp.hi))))
         if static and not B.edge:
             for i, (m, x) in enumerate(zip(maps, xs)):
+                if x is None:
+                    continue
                 B.need_span(x[2], B.bound(f.domain[i].lowerBound), B.bound(f.domain[i].upperBound))
                 for b in m.lows:
                     B.need_ge(x[2], x[2].lo, B.bound(b))
@@ -267,18 +281,22 @@ class _Item(object):
                     B.need_le(x[2], x[2].hi, B.bound(b))
         if static:
             # scalar base of the row: every constant but the innermost's
-            key = (f.name, tuple((x[2].d, x[2].A, x[0] if i < nd - 1 else 0) for i, x in enumerate(xs)))
+            key = (f.name, tuple((x[2].d, x[2].A, x[0] if i < nd - 1 else 0) if x is not None else None
+                                 for i, x in enumerate(xs)))
             if key not in B.uni:
                 nm = 'gp%d' % len(B.uni)
                 terms = []
-                for i, (d, A, c) in enumerate(key[1]):
+                for i, k in enumerate(key[1]):
+                    if k is None:
+                        continue
+                    d, A, c = k
                     e = '(%s)' % B.coord(Span(d, A, 0, 0), c)
                     terms.append('(%s - LB_%s_%d)%s' % (e, f.name, i, ' * S_%s_%d' % (f.name, i) if i < nd - 1 else ''))
                 B.uni[key] = nm
                 B.uni_lines.append('const auto %s = G_%s + (%s);' % (nm, f.name, ' + '.join(terms) or '0'))
             coef = {}
             for i, x in enumerate(xs):
-                for k, st in x[1].items():
+                for k, st in (x[1] if x is not None else {}).items():
                     coef.setdefault(k, []).append((st, 'S_%s_%d' % (f.name, i) if i < nd - 1 else None))
             okey = ('g', f.typ.nbytes(), tuple(sorted((k, tuple(v)) for k, v in coef.items())))
 
@@ -289,8 +307,8 @@ class _Item(object):
                         terms.append('(unsigned)j%d * %s' % (k, '(unsigned)(%s * %d)' % (S, st) if S else '%du' % st))
                 return 'const unsigned %s = (%s) * %du;' % (n, ' + '.join(terms) or '0u', f.typ.nbytes())
             off = self.base(okey, mk)
-            c = xs[-1][0] if nd else 0
-            fast = 'pmx_at(%s, %s)[%d]' % (B.uni[key], off, c)
+            c = xs[-1][0] if nd and xs[-1] is not None else 0
+            fast = 'pmx_at(%s, %s)[%d]' % (B.uni[key], ' + '.join([off] + dyn), c)
             if not B.edge:
                 return fast
             ekey = (key, okey, c)
