@@ -69,10 +69,10 @@ def unsharp(rows=2848, cols=4256, tiles=(32, 256), gpu_options=None, with_data=T
     pd = {}
     out = unsharp_mask_full(pd)
     R, C = rows - 4, cols - 4
-    # the mask's blocks one row tall: twice the items of the 2x4 blocks the
-    # planner's estimate picks, for memory latency (61.0 -> 60.3 us at
-    # 3 x 2848 x 4256)
-    gpu_options = dict({'box_blocks': {'mask': [1, 4]}}, **(gpu_options or {}))
+    # the general kernel: at 12 MPix both are bound by memory (60.8 and
+    # 61.1 us), on a 170 x 200 image the box kernel's longer prologue shows
+    # (3.6 and 4.1 us)
+    gpu_options = dict({'no_box': 1}, **(gpu_options or {}))
     pipe = _pipe(out, pd, {'R': R, 'C': C}, 'unsharp', list(tiles), group_size,
                  gpu_options=gpu_options, literal_mode=literal_mode)
     vals = {'R': R, 'C': C, 'threshold': 0.001, 'weight': 3.0}
