@@ -787,7 +787,7 @@ def _stores(B, item, m, mi, pts, SL):
 
 def emit_box_kernel(pipe, plan, kname, threads, mode, xcd=True):
     """(HIP source, KernelInfo) of one box kernel."""
-    from .hip_emit import (KernelInfo, wrap_kernel, group_buffers, tile_lines, stride_lines, grid_exprs)
+    from .hip_emit import (KernelInfo, _prod, wrap_kernel, group_buffers, tile_lines, stride_lines, grid_exprs)
     params = pipe.sorted_parameters()
     reads, writes, buffers = group_buffers(plan)
     L = []
@@ -859,4 +859,8 @@ def emit_box_kernel(pipe, plan, kname, threads, mode, xcd=True):
     grid_c, tiles_c = grid_exprs(plan, base_pr, 1)
     info = KernelInfo(kname, 'group', buffers, grid_c, threads, plan.lds_bytes, plan, reads, writes)
     info.tiles_c = tiles_c
+    tiles = 1
+    for n in plan.tile_space():
+        tiles *= n
+    info.work = tiles * sum(_prod([sp.ext for sp in s.span]) for s in plan.stages if not s.inline)
     return wrap_kernel(kname, params, buffers, writes, threads, plan.lds_bytes, L), info

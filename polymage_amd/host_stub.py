@@ -84,7 +84,9 @@ def _validation_lines(pipe, pr):
     return lines
 
 
-def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_PATH@'):
+def emit_host_stub(pipe, kernels, launches, host_consts, co_symbol='pmx_co', co_path='@CO_PATH@'):
+    """``kernels``: every kernel, for the batch API; ``launches``: the plain
+    launches of one call, in order (kernels, or several merged into one)."""
     pr = Printer({}, None, pipe.literal_mode)
     name = pipe.name
     params = pipe.sorted_parameters()
@@ -109,17 +111,20 @@ def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_
     w('extern "C" const unsigned char %s_image[];' % co_symbol)
     w('__asm__(".section .rodata\\n.balign 64\\n.global %s_image\\n%s_image:\\n.incbin \\"%s\\"\\n.byte 0\\n.previous\\n");'
       % (co_symbol, co_symbol, co_path))
+    nl = len(launches)
     w('static const char* pmx_kernel_names[%d] = {%s};' % (
         max(1, nk), ', '.join('"%s"' % k.name for k in kernels) or '""'))
+    w('static const char* pmx_launch_names[%d] = {%s};' % (
+        max(1, nl), ', '.join('"%s"' % k.name for k in launches) or '""'))
     w('static void* pmx_mod[64];')
-    w('static void* pmx_fn[64][%d];' % max(1, nk))
+    w('static void* pmx_fn[64][%d];' % max(1, nl))
     w('static void* pmx_fn_batch[64][%d];' % max(1, nk))
     w('static int pmx_load(int dev) {')
     w('  if (dev < 0 || dev >= 64) { pmx_set_error("device index"); return -1; }')
     w('  if (pmx_mod[dev]) return 0;')
     w('  void* m = nullptr;')
     w('  int rc = pmx_module_load_data(%s_image, &m); if (rc) return rc;' % co_symbol)
-    w('  for (int k = 0; k < %d; ++k) { rc = pmx_module_function(m, pmx_kernel_names[k], &pmx_fn[dev][k]); if (rc) return rc; }' % nk)
+    w('  for (int k = 0; k < %d; ++k) { rc = pmx_module_function(m, pmx_launch_names[k], &pmx_fn[dev][k]); if (rc) return rc; }' % nl)
     w('  for (int k = 0; k < %d; ++k) { char nm[256]; snprintf(nm, sizeof nm, "%%s_batch", pmx_kernel_names[k]); '
       'rc = pmx_module_function(m, nm, &pmx_fn_batch[dev][k]); if (rc) return rc; }' % nk)
     w('  pmx_mod[dev] = m;')
@@ -170,7 +175,7 @@ def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_
           % (name, f.name, _size(f, pr), c_type(f.typ), b))
         bufname[f] = b
     w('  void* pmx_err = nullptr; rc = pmx_arena_get_zeroed("%s/err", 64, &pmx_err); if (rc) return rc;' % name)
-    _launch_lines(w, kernels, params, bufname)
+    _launch_lines(w, launches, params, bufname)
     w('  return 0;')
     w('}')
 
@@ -216,7 +221,7 @@ def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_
         f = cp.func
         w('  rc = pmx_memcpy_h2d(b_%s, h_%s, n_%s, stream); if (rc) return rc;' % (f.name, f.name, f.name))
     w('  void* pmx_err = pmx_scr;')
-    _launch_lines(w, kernels, params, nb)
+    _launch_lines(w, launches, params, nb)
     w('  return 0;')
     w('}')
 
@@ -263,7 +268,7 @@ def emit_host_stub(pipe, kernels, host_consts, co_symbol='pmx_co', co_path='@CO_
 
 
 def _launch_lines(w, kernels, params, bufname):
-    """One launch per kernel, in order, on ``stream``; ``pmx_err``, ``dev``
+    """The launches, in order, on ``stream``; ``pmx_err``, ``dev``
     and ``rc`` are in scope."""
     for k in kernels:
         w('  {')
@@ -274,6 +279,9 @@ def _launch_lines(w, kernels, params, bufname):
         for p in params:
             w('    %s a_%s = %s;' % (c_type(p.typ), p.name, p.name))
             argv.append('&a_%s' % p.name)
+        for i, m in enumerate(k.members or ()):
+            w('    int n_%d = (int)std::max<long long>(0, %s);' % (i, m.grid_c))
+            argv.append('&n_%d' % i)
         w('    void* args[] = {%s};' % (', '.join(argv) or 'nullptr'))
         w('    long long grid = %s;' % k.grid_c)
         w('    if (grid > 0) { rc = pmx_launch(pmx_fn[dev][%d], (unsigned)grid, 1, 1, %d, 1, 1, 0, stream, args); if (rc) return rc; }'

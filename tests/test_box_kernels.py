@@ -179,3 +179,48 @@ def test_batch_of_many_frames(gpu, n):
             assert all(bits_equal(d['harris'].cpu().numpy(), r) for d, r in zip(dev, refs))
     finally:
         bp.batch_destroy(h)
+
+
+def test_merged_launches_keep_dependences():
+    """Every kernel is launched once, after what it reads, and never beside a
+    kernel that writes what it reads; merged members have equal workgroups."""
+    from polymage_amd.apps import workloads
+    from polymage_amd.hip_emit import plan_launches
+    for app in ('blend', 'laplacian', 'interpolate', 'bilateral'):
+        w = workloads.tuned(app, 'learned', with_data=False)
+        kernels = w.pipe.generate_code().kernels
+        launches = plan_launches(w.pipe, kernels, w.pipe.sorted_parameters())[1]
+        written = dict((f, k) for k in kernels for f in k.writes)
+        done = []
+        for l in launches:
+            members = l.members or [l]
+            assert len(set(m.threads for m in members)) == 1
+            for m in members:
+                for f in m.reads:
+                    assert f not in written or written[f] in done
+            done += members
+        assert len(done) == len(kernels) and set(done) == set(kernels)
+        if app in ('blend', 'laplacian'):
+            assert len(launches) < len(kernels)
+
+
+def _blend(opts):
+    from polymage_amd.apps.pyramid_blend import pyramid_blend
+    pd = {}
+    out = pyramid_blend(pd)
+    R, C = 130, 203
+    g = np.random.default_rng(3)
+    pipe = build(out, pd, {'R': R, 'C': C}, 'blend', [8, 64], group_size=6, gpu_options=opts)
+    return out, pipe, {'R': R, 'C': C, 'img1': g.random((3, R, C)).astype(np.float32),
+                       'img2': g.random((3, R, C)).astype(np.float32),
+                       'mask': g.random((R, C)).astype(np.float32)}, (3, R - 60, C - 60)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opts", [None, {'no_merge': 1}])
+def test_merged_launches_bitexact(gpu, opts):
+    if emulating():
+        pytest.skip("the emulator's blend tests run merged launches")
+    print("case merged", opts, flush=True)
+    out, pipe, vals, shape = _blend(opts)
+    _check(out, gpu_build(pipe).run_host, vals, shape)
