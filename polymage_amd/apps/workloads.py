@@ -242,7 +242,7 @@ BUILDERS = {'harris': harris, 'unsharp': unsharp, 'bilateral': bilateral,
 
 def schedule(app, which='learned'):
     """(tiles, group_size, gpu_options, label) of ``app`` under the
-    autotuner's recorded pick ('learned' or 'exhaustive', from
+    recorded pick ('learned' or 'exhaustive', from
     polymage_amd/tuned.json) or the default tiles ('default', or when no
     pick is recorded)."""
     from .. import tuner
@@ -252,7 +252,9 @@ def schedule(app, which='learned'):
     gopts = {'threads': rec['threads']}
     if rec.get('lanes'):
         gopts['lanes'] = 1
-    return tuple(rec['tiles']), rec['group_size'], gopts, '%s: %s' % (which, rec['key'])
+    gopts.update(rec.get('batch') or {})
+    return tuple(rec['tiles']), rec['group_size'], gopts, '%s: %s' % ('swept' if rec['swept'] else which,
+                                                                      rec['key'])
 
 
 def class_schedules(app, which='learned'):

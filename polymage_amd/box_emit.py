@@ -785,7 +785,7 @@ def _stores(B, item, m, mi, pts, SL):
             w('if (%s) %s' % (' && '.join(c), x) if c else x)
 
 
-def emit_box_kernel(pipe, plan, kname, threads, mode, xcd=True):
+def emit_box_kernel(pipe, plan, kname, threads, mode, xcd=True, forms=('plain', 'batch')):
     """(HIP source, KernelInfo) of one box kernel."""
     from .hip_emit import (KernelInfo, _prod, wrap_kernel, group_buffers, tile_lines, stride_lines, grid_exprs)
     params = pipe.sorted_parameters()
@@ -863,4 +863,4 @@ def emit_box_kernel(pipe, plan, kname, threads, mode, xcd=True):
     for n in plan.tile_space():
         tiles *= n
     info.work = tiles * sum(_prod([sp.ext for sp in s.span]) for s in plan.stages if not s.inline)
-    return wrap_kernel(kname, params, buffers, writes, threads, plan.lds_bytes, L), info
+    return wrap_kernel(kname, params, buffers, writes, threads, plan.lds_bytes, L, forms), info

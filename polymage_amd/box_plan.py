@@ -361,7 +361,7 @@ class BoxPlan(GroupPlan):
         if o.get('no_box') or any(o.get(k) for k in GENERAL_ONLY) or int(o.get('roll', 1)) > 1:
             return None
         try:
-            return BoxPlan(plan.pipe, plan.group, plan.gindex)
+            return BoxPlan(plan.pipe, plan.group, plan.gindex, plan.tile_sizes, plan.opts)
         except PlanError:
             return None
 

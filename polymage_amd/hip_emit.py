@@ -40,6 +40,9 @@ def _prod(xs):
     return n
 
 
+# entry points a kernel's source can carry: its plain body, its batch form
+FORMS = ('plain', 'batch')
+
 # separators of the two parts in the printed source (runtime.split_source)
 HIP_MARK = '// ===== HIP kernels (hiprtc, gfx950) =====\n'
 HOST_MARK = '\n// ===== host stub (g++) =====\n'
@@ -185,7 +188,7 @@ def grid_exprs(plan, base_pr, roll):
     return grid_c, tiles_c
 
 
-def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
+def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True, forms=FORMS):
     """HIP source of one stencil-group kernel."""
     params = pipe.sorted_parameters()
     stages = plan.stages
@@ -918,7 +921,7 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True):
     info.tiles_c = tiles_c
     info.roll = roll
     info.work = plan.total_tiles * sum(_prod(s.static_ext) for s in stages if not s.inline)
-    return wrap_kernel(kname, params, buffers, writes, threads, plan.lds_bytes, L), info
+    return wrap_kernel(kname, params, buffers, writes, threads, plan.lds_bytes, L, forms), info
 
 
 
@@ -1175,7 +1178,7 @@ def kernel_args(params, buffers, writes):
     return decls, names, fields
 
 
-def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines):
+def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines, forms=FORMS):
     """The kernel body as a device function (its plain entry point, one
     workgroup per tile, is plain_kernel's or merged_kernel's) and the batch
     entry point:
@@ -1199,10 +1202,14 @@ def wrap_kernel(kname, params, buffers, writes, threads, lds_bytes, body_lines):
     prologue = '  (void)pmx_remap; (void)pmx_lds; (void)pmx_err; (void)pmx_rk; (void)pmx_rr;'
     # plain form: kernel arguments, whose address space and aliasing the
     # compiler knows, and the thread index with its known range
-    L = ['__device__ __forceinline__ void %s_body(%s) {' % (kname, ', '.join(decls + tail)),
-         prologue, '  const int pmx_tx = (int)threadIdx.x; (void)pmx_tx;']
-    L += body_lines
-    L.append('}')
+    L = []
+    if 'plain' in forms:
+        L += ['__device__ __forceinline__ void %s_body(%s) {' % (kname, ', '.join(decls + tail)),
+              prologue, '  const int pmx_tx = (int)threadIdx.x; (void)pmx_tx;']
+        L += body_lines
+        L.append('}')
+    if 'batch' not in forms:
+        return '\n'.join(L) + '\n'
     # batch form: the same body over pointers read from frame records.
     # Buffers the kernel writes are global-address-space pointers (global,
     # not flat, stores); buffers it only reads are constant-address-space
@@ -1361,16 +1368,34 @@ def plan_pipeline(pipe):
     return plans
 
 
-def _emit_group(pipe, plan, kname, threads, mode, xcd):
+def _emit_group(pipe, plan, kname, threads, mode, xcd, forms=FORMS):
     """The box kernel of a group that has constant boxes, else the general
     kernel."""
     box = BoxPlan.of(plan)
     if box is not None:
         try:
-            return emit_box_kernel(pipe, box, kname, threads, mode, xcd)
+            return emit_box_kernel(pipe, box, kname, threads, mode, xcd, forms)
         except PlanError:
             pass
-    return emit_group_kernel(pipe, plan, kname, threads, mode, xcd)
+    return emit_group_kernel(pipe, plan, kname, threads, mode, xcd, forms)
+
+
+def _batch_plan(pipe, plan, opts):
+    """The plan of a group's batch form under gpu option ``batch_tiles`` (and
+    ``batch_threads``), or None: its plain form serves both.
+
+    A single frame wants many small tiles, enough workgroups for 256 compute
+    units; a batch has workgroups to spare and wants large ones, which
+    compute less twice (camera pipe: 1216 x 1664 21.7 us with 32 x 32 tiles and
+    23.4 with 32 x 64, 48 frames 869 and 640)."""
+    tiles = opts.get('batch_tiles')
+    if not tiles or not isinstance(plan, GroupPlan):
+        return None
+    try:
+        return GroupPlan(pipe, plan.group, plan.gindex, list(tiles),
+                         {'threads': int(opts.get('batch_threads', opts.get('threads', 256)))})
+    except PlanError:
+        return None
 
 
 def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
@@ -1382,15 +1407,23 @@ def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
     srcs = ['// generated by polymage_amd for pipeline %s' % pipe.name,
             DEVICE_PRELUDE, REGION_PRELUDE, BOX_PRELUDE]
     kernels = []
+    batch = []          # the kernels of the batch API
     host_consts = []
     for i, plan in enumerate(plans):
         kname = 'pmx_%s_g%d' % (pipe.name, i)
+        bplan = _batch_plan(pipe, plan, opts)
+        if bplan is not None:
+            src, info = _emit_group(pipe, bplan, kname + 'b', int(bplan.opts['threads']), mode, xcd, ('batch',))
+            srcs.append(src)
+            batch.append(info)
         if isinstance(plan, GroupPlan):
-            src, info = _emit_group(pipe, plan, kname, threads, mode, xcd)
+            src, info = _emit_group(pipe, plan, kname, threads, mode, xcd,
+                                    FORMS if bplan is None else ('plain',))
         elif isinstance(plan, ReductionPlan):
             for src, info in emit_reduction_kernel(pipe, plan, kname, mode):
                 srcs.append(src)
                 kernels.append(info)
+                batch.append(info)
             continue
         else:
             if plan.on_host:
@@ -1399,9 +1432,11 @@ def emit_pipeline(pipe, is_extern_c_func=True, are_io_void_ptrs=True):
             src, info = emit_const_kernel(pipe, plan, kname, mode)
         srcs.append(src)
         kernels.append(info)
+        if bplan is None:
+            batch.append(info)
     plain, launches = plan_launches(pipe, kernels, pipe.sorted_parameters())
     hip_src = '\n'.join(srcs + plain)
     from .host_stub import emit_host_stub
-    host_src = emit_host_stub(pipe, kernels, launches, host_consts)
+    host_src = emit_host_stub(pipe, kernels, launches, batch, host_consts)
     return GeneratedCode(pipe.name, hip_src, host_src, kernels,
                          {'plans': plans, 'threads': threads})

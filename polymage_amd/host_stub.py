@@ -84,15 +84,16 @@ def _validation_lines(pipe, pr):
     return lines
 
 
-def emit_host_stub(pipe, kernels, launches, host_consts, co_symbol='pmx_co', co_path='@CO_PATH@'):
-    """``kernels``: every kernel, for the batch API; ``launches``: the plain
-    launches of one call, in order (kernels, or several merged into one)."""
+def emit_host_stub(pipe, kernels, launches, batch, host_consts, co_symbol='pmx_co', co_path='@CO_PATH@'):
+    """``kernels``: every kernel of a call; ``launches``: its launches, in
+    order (kernels, or several merged into one); ``batch``: the kernels of
+    the batch API."""
     pr = Printer({}, None, pipe.literal_mode)
     name = pipe.name
     params = pipe.sorted_parameters()
     inputs = pipe.sorted_inputs()
     outputs = pipe.sorted_outputs()
-    nk = len(kernels)
+    nk = len(batch)
     L = []
     w = L.append
     w('// host stub for pipeline %s (generated)' % name)
@@ -112,8 +113,8 @@ def emit_host_stub(pipe, kernels, launches, host_consts, co_symbol='pmx_co', co_
     w('__asm__(".section .rodata\\n.balign 64\\n.global %s_image\\n%s_image:\\n.incbin \\"%s\\"\\n.byte 0\\n.previous\\n");'
       % (co_symbol, co_symbol, co_path))
     nl = len(launches)
-    w('static const char* pmx_kernel_names[%d] = {%s};' % (
-        max(1, nk), ', '.join('"%s"' % k.name for k in kernels) or '""'))
+    w('static const char* pmx_batch_names[%d] = {%s};' % (
+        max(1, nk), ', '.join('"%s"' % k.name for k in batch) or '""'))
     w('static const char* pmx_launch_names[%d] = {%s};' % (
         max(1, nl), ', '.join('"%s"' % k.name for k in launches) or '""'))
     w('static void* pmx_mod[64];')
@@ -125,7 +126,7 @@ def emit_host_stub(pipe, kernels, launches, host_consts, co_symbol='pmx_co', co_
     w('  void* m = nullptr;')
     w('  int rc = pmx_module_load_data(%s_image, &m); if (rc) return rc;' % co_symbol)
     w('  for (int k = 0; k < %d; ++k) { rc = pmx_module_function(m, pmx_launch_names[k], &pmx_fn[dev][k]); if (rc) return rc; }' % nl)
-    w('  for (int k = 0; k < %d; ++k) { char nm[256]; snprintf(nm, sizeof nm, "%%s_batch", pmx_kernel_names[k]); '
+    w('  for (int k = 0; k < %d; ++k) { char nm[256]; snprintf(nm, sizeof nm, "%%s_batch", pmx_batch_names[k]); '
       'rc = pmx_module_function(m, nm, &pmx_fn_batch[dev][k]); if (rc) return rc; }' % nk)
     w('  pmx_mod[dev] = m;')
     w('  return 0;')
@@ -258,7 +259,7 @@ def emit_host_stub(pipe, kernels, launches, host_consts, co_symbol='pmx_co', co_
     w('  rc = pmx_stream_sync(nullptr); if (rc) return rc;')
     w('  return pipeline_%s_status();' % name)
     w('}')
-    _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None)
+    _emit_batch_api(pipe, batch, host_consts, L, pr)
     w('extern "C" void pipeline_%s(%s) {' % (name, ', '.join(hsig)))
     w('  int rc = pipeline_%s_host(%s);' % (name, ', '.join(
         [p.name for p in params] + ['%s_void_arg' % f.name for f in inputs + outputs])))
@@ -301,7 +302,7 @@ def frame_struct_fields(kernel, params):
     return fields, size
 
 
-def _emit_batch_api(pipe, kernels, host_consts, L, pr, bufname_fn=None):
+def _emit_batch_api(pipe, kernels, host_consts, L, pr):
     """Batched execution of many frames of different sizes.
 
     pipeline_<name>_batch_create(n, per-frame parameter arrays...,

@@ -617,9 +617,11 @@ def parse_key(key):
 
 
 def tuned_schedule(app, which='learned', path=None):
-    """The schedule the autotuner recorded for ``app`` ('learned': the cost
-    model's best timed top-k candidate; 'exhaustive': the exhaustive best),
-    or None."""
+    """The schedule recorded for ``app``, or None.  'exhaustive': the
+    exhaustive search's best.  'learned': the pick of a sweep over several
+    frame sizes where one is recorded (``swept_best``, and ``swept_batch`` for
+    the batch form's tiles: the searches time one full-size frame, with the
+    general kernels), else the cost model's best timed top-k candidate."""
     path = path or TUNED_PATH
     if not os.path.exists(path):
         return None
@@ -628,4 +630,12 @@ def tuned_schedule(app, which='learned', path=None):
     if not rec:
         return None
     key = rec.get('learned_best' if which == 'learned' else 'exhaustive_best')
-    return parse_key(key) if key else None
+    swept = rec.get('swept_best') if which == 'learned' else None
+    if not (swept or key):
+        return None
+    out = parse_key(swept or key)
+    out['swept'] = bool(swept)
+    if swept and rec.get('swept_batch'):
+        b = parse_key(rec['swept_batch'])
+        out['batch'] = {'batch_tiles': list(b['tiles']), 'batch_threads': b['threads']}
+    return out

@@ -224,3 +224,25 @@ def test_merged_launches_bitexact(gpu, opts):
     print("case merged", opts, flush=True)
     out, pipe, vals, shape = _blend(opts)
     _check(out, gpu_build(pipe).run_host, vals, shape)
+
+
+@pytest.mark.parametrize("opts", [{'batch_tiles': [16, 48]}, {'batch_tiles': [32, 64], 'batch_threads': 128},
+                                  {'batch_tiles': [512, 512]}])
+def test_batch_tiles_on_the_emulator(opts):
+    """Batch kernels on tiles of their own (the last do not fit LDS: the
+    plain kernels' tiles serve the batch) give the plain call's output."""
+    import kernel_emu
+    sizes = [(114, 162), (128, 192), (98, 130)]
+    recs, refs = [], []
+    for (R, C) in sizes:
+        out, pipe, vals, shape = _app('campipe', R, C, [16, 32], opts)
+        o = np.full(shape, 7, np.uint8)
+        cemit.build([out], 'box_process')(dict(vals, process=o))
+        refs.append(o)
+        recs.append(dict(vals, process=np.full(shape, 7, np.uint8)))
+    ep = kernel_emu.build(pipe)
+    ep.run_batch(recs, 'persistent')
+    assert all(bits_equal(rec['process'], r) for rec, r in zip(recs, refs))
+    g = np.full(shape, 7, np.uint8)
+    ep.run_host(dict(vals, process=g))
+    assert bits_equal(g, refs[-1])
