@@ -763,7 +763,15 @@ class BoxPlan(GroupPlan):
             dyn = any(m.kind == '*' or (m.kind == 'var' and blk[m.dim] % m.period and m.period > 1)
                       for m in ms)
             if dyn:
-                total += 5.0 * len(pts)
+                # a sum per computed index and point; an index that varies
+                # along one dimension only is computed once per row of it.
+                # (A bilateral slice reads one grid row for 8 rows of pixels:
+                # 8x1 points a thread share it, 4x2 compute it 4 times; on
+                # 64x64 tiles 33.6 against 29.4 us for 2560x1536.)
+                along = set(m.dim for m in ms if m.kind == 'var' and
+                            m.period > 1 and blk[m.dim] % m.period)
+                total += (3.0 + len(along) + any(m.kind == '*' for m in ms)) * len(pts)
+                total += 3.0 * sum(blk[i] for i in along)
                 continue
             seen = runs.setdefault((r.objectRef, tuple((m.kind, m.dim, m.slope) for m in ms)), set())
             for u in pts:
