@@ -308,7 +308,7 @@ class Printer(object):
     text of a Reference, ``var_names`` maps Variables to C names."""
 
     def __init__(self, var_names, ref_cb, mode='double', param_prefix='', lazy=False,
-                 exact_fma=False, unify=None):
+                 exact_fma=False, unify=None, minmax=True):
         self.var_names = var_names
         self.ref_cb = ref_cb
         self.mode = mode
@@ -321,6 +321,8 @@ class Printer(object):
         # SelectUnifier when only index arithmetic is left to select;
         # ``unify`` is its cheap_ref test (None: off)
         self.unify = unify
+        # Min, Max and their like through the device helpers
+        self.minmax = minmax
         self._tmp = [0]
 
     def tmp(self):
@@ -367,7 +369,7 @@ class Printer(object):
                 if u is not None and not isinstance(u, CSelect) and uf.index_only(u):
                     return '((%s)(%s))' % (c_type(getType(e)), self.expr(u, pro))
             if self.lazy and pro is not None:
-                m = self._minmax(e)
+                m = self._minmax(e) if self.minmax else None
                 if m is not None:
                     # both operands are compared and so always run: as
                     # arguments they are read once, where a conditional

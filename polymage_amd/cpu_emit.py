@@ -202,7 +202,7 @@ class _Emitter(object):
 
         def stage_value(s, target, pnames, i0, skip_single):
             vn = dict(zip(s.func.variables, pnames))
-            pr = Printer(vn, make_cb(s), mode, lazy=True)
+            pr = Printer(vn, make_cb(s), mode, lazy=True, minmax=False)
             single = len(s.parts) == 1
             for pi, part in enumerate(s.parts):
                 conds = []
@@ -327,7 +327,7 @@ class _Emitter(object):
             w('for (int f%d = %s; f%d <= %s; ++f%d) {' % (d, base.expr(f.domain[d].lowerBound), d,
                                                          base.expr(f.domain[d].upperBound), d), i0)
             i0 += 1
-        dpr = Printer(dict((plan.fvars[d], 'f%d' % d) for d in range(nd)), cb, mode, lazy=True)
+        dpr = Printer(dict((plan.fvars[d], 'f%d' % d) for d in range(nd)), cb, mode, lazy=True, minmax=False)
         pro = []
         dv = dpr.expr(f.default, pro)
         for l in pro:
@@ -342,7 +342,7 @@ class _Emitter(object):
                 j, base.expr(f.reductionDomain[j].lowerBound), j,
                 base.expr(f.reductionDomain[j].upperBound), j), i0)
             i0 += 1
-        pr = Printer(dict(zip(plan.rvars, rnames)), cb, mode, lazy=True)
+        pr = Printer(dict(zip(plan.rvars, rnames)), cb, mode, lazy=True, minmax=False)
         for rc in plan.cases:
             red = rc.red
             w('{', i0)
@@ -364,7 +364,7 @@ class _Emitter(object):
                     if v not in plan.rvars:
                         vn[v] = '(%s)' % tn[d]
                 cpro = []
-                cond = Printer(vn, cb, mode, lazy=True).cond(rc.cond, cpro)
+                cond = Printer(vn, cb, mode, lazy=True, minmax=False).cond(rc.cond, cpro)
                 for l in cpro:
                     w(l, i0 + 1)
             slot = 'G_%s[%s]' % (f.name, _gindex(f, tn, base))
@@ -396,7 +396,7 @@ class _Emitter(object):
             g = ref.objectRef
             idx = [pr.expr(a, pro) for a in ref.arguments]
             return 'G_%s[%s]' % (g.name, _gindex(g, idx, base))
-        pr = Printer(dict(zip(f.variables, names)), cb, mode, lazy=True)
+        pr = Printer(dict(zip(f.variables, names)), cb, mode, lazy=True, minmax=False)
         w('{ // const %s' % f.name)
         i0 = 1
         for i in range(nd):
