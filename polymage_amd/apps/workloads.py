@@ -88,7 +88,8 @@ def bilateral(rows=2560, cols=1536, tiles=(32, 64), gpu_options=None, with_data=
     from .bilateral import bilateral_grid_full
     pd = {}
     out = bilateral_grid_full(pd)
-    # the slice's blocks without 128-bit LDS row loads (48.1 -> 47.6 us)
+    # general kernels: the slice's blocks without 128-bit LDS row loads
+    # (48.1 -> 47.6 us; box kernels choose their own)
     gpu_options = dict({'no_vlds': 1}, **(gpu_options or {}))
     pipe = _pipe(out, pd, {'rows': rows, 'cols': cols}, 'bilateral', list(tiles), group_size,
                  gpu_options=gpu_options, literal_mode=literal_mode)
@@ -123,7 +124,8 @@ def laplacian(rows=2560, cols=1536, tiles=(32, 64), gpu_options=None, with_data=
     # K times the LDS still leaves several workgroups per CU
     # (148.8 -> 141.2 us per call at the learned schedule); with that, the
     # larger per-thread blocks of a higher fixed cost per sweep iteration
-    # in the block choice (141.2 -> 139.6 us)
+    # in the general kernels' block choice (141.2 -> 139.6 us; box kernels,
+    # which ignore it, 106.9)
     kgroups = dict(('D_gPyramid_L%d' % j if j > 1 else 'gPyramid_L0', [8, 16])
                    for j in range(1, min(J, 4)))
     gpu_options = dict({'kblock': 1, 'group_tiles': kgroups, 'iter_cost': 10},
@@ -145,8 +147,8 @@ def campipe(rows=1216, cols=1664, tiles=(16, 64), gpu_options=None, with_data=Tr
     from .campipe import camera_pipe, MATRIX_3200, MATRIX_7000
     pd = {}
     out = camera_pipe(pd, variant='batch')
-    # the largest per-thread blocks the sweeps allow (a high fixed cost per
-    # sweep iteration in the block choice): its 26 stages each pay a loop
+    # general kernels: the largest per-thread blocks the sweeps allow (a high
+    # fixed cost per sweep iteration in the block choice): its 26 stages each pay a loop
     # guard and a fast/slow split per item (48-frame batch 1.48 -> 1.44 ms)
     gpu_options = dict({'iter_cost': 80}, **(gpu_options or {}))
     pipe = _pipe(out, pd, {'R': rows, 'C': cols}, 'campipe', list(tiles), group_size,
@@ -202,7 +204,8 @@ def blend(rows=2560, cols=1536, tiles=(16, 64), gpu_options=None, with_data=True
     out = pyramid_blend(pd)
     R, C = rows, cols
     # smaller per-thread blocks than the default choice (a low fixed cost
-    # per sweep iteration in the block choice): 207 -> 201 us per call
+    # per sweep iteration in the general kernels' block choice):
+    # 207 -> 201 us per call
     gpu_options = dict({'iter_cost': 3}, **(gpu_options or {}))
     pipe = _pipe(out, pd, {'R': R, 'C': C}, 'blend', list(tiles), group_size,
                  gpu_options=gpu_options, literal_mode=literal_mode)

@@ -52,7 +52,7 @@ def _workload(app):
 
 
 # size-class specs -> the frames of the class: such a spec is timed as one
-# persistent launch over the class's frames (the batch it will run), not
+# batch launch over the class's frames (the batch it will run), not
 # as a single frame's plain launch
 _CLASS_FRAMES = {}
 
@@ -156,7 +156,7 @@ def size_class_specs(spec):
     of the application's benchmark batch (the camera pipeline's 48 seeded
     frames) and the spec of each class's representative frame.  Each
     class's candidates are planned at the representative size and timed as
-    a persistent batch launch over the class's own frames."""
+    a batch launch over the class's own frames."""
     from .apps import inputs
     from .size_classes import frame_classes
     app, k = spec.split(':')

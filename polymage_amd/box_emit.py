@@ -18,8 +18,7 @@ multiples of the chunk, so its alignment is known at compile time.
 """
 
 from .analysis import PlanError
-from .box_plan import BoxPlan, Known, Span, arg_map, const_int, fold
-from .constructs import Reference
+from .box_plan import Known, Span, arg_map, const_int, fold
 from .cprint import Printer, c_type
 from .region_ir import bound_c
 

@@ -39,7 +39,7 @@ from .expr_ast import (AbstractBinaryOpNode, AbstractUnaryOpNode, Value, Paramet
                        Condition, Select, Cast, InbuiltFunction)
 from .expr_types import Int
 from .expression import substitute_vars, substitute_refs, getType, _rebuild_bin
-from .group_plan import GroupPlan, StageInfo, LDS_LIMIT_BYTES
+from .group_plan import GroupPlan, StageInfo
 
 # gpu options that ask for a particular form of the general kernel
 GENERAL_ONLY = ('block', 'block_lds', 'lanes', 'stage', 'no_inline', 'no_fuse', 'index64',

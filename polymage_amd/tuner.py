@@ -577,7 +577,7 @@ def time_batch(bp, workload, frames, frame_input='img', runs=5, warmup=1, reps=3
 
 def time_candidates_batch(workload, compiled, frames, runs=5, db=None, app=None, verbose=False):
     """time_candidates with a batch of frames as the objective (the
-    persistent launch over all of them, ``time_batch``); returns {key: ms}."""
+    batch launch over all of them, ``time_batch``); returns {key: ms}."""
     w = workload(rows=frames[0].shape[0], cols=frames[0].shape[1], with_data=False)
     mpix = 0.0
     out = {}
