@@ -18,7 +18,7 @@ multiples of the chunk, so its alignment is known at compile time.
 """
 
 from .analysis import PlanError
-from .box_plan import Known, Span, arg_map, const_int, fold
+from .box_plan import Known, Span, arg_map, const_int, fold, least_values
 from .cprint import Printer, c_type
 from .region_ir import bound_c
 
@@ -420,7 +420,8 @@ class _Item(object):
 
         def assign(part, i):
             pro = []
-            val = pr.expr(fold(part.expr, kt), pro)
+            kp = Known(kt.value, kt.mod, least_values(t.func, part))
+            val = pr.expr(fold(part.expr, kp), pro)
             for l in pro:
                 w(l, i)
             w('%s = %s;%s' % (target, val, ' pmx_w = true;' if flag else ''), i)

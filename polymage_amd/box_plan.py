@@ -197,11 +197,23 @@ def image(m, span):
 
 class Known(object):
     """What is known of a stage's variables at one point of a block:
-    ``value[v]`` an integer, or ``mod[v]`` = (modulus, residue)."""
+    ``value[v]`` an integer, or ``mod[v]`` = (modulus, residue); ``least[v]``
+    a lower bound of v over the points that count (``least_values``)."""
 
-    def __init__(self, value, mod):
+    def __init__(self, value, mod, least=None):
         self.value = value
         self.mod = mod
+        self.least = least or {}
+
+
+def least_values(func, part):
+    """{variable: constant lower bound} over the points of a Case part."""
+    out = {}
+    for v, dom, (lo, _) in zip(func.variables, func.domain, part.box):
+        bounds = [b for b in (const_int(dom.lowerBound), const_int(lo)) if b is not None]
+        if bounds:
+            out[v] = max(bounds)
+    return out
 
 
 def _ival(e):
@@ -222,20 +234,30 @@ def decide(c, kn):
     return {'==': l == r, '!=': l != r, '<': l < r, '<=': l <= r, '>': l > r, '>=': l >= r}[c.conditional]
 
 
-def _residue(e, kn):
-    """(modulus, residue) of an integer expression v + c, else None."""
+def _shifted(e):
+    """(variable, c) of an expression v + c, else None."""
     e = Value.numericToValue(e)
     if isinstance(e, Variable):
-        return kn.mod.get(e)
+        return e, 0
     if isinstance(e, AbstractBinaryOpNode) and e.op in ('+', '-'):
         l, r = Value.numericToValue(e.left), Value.numericToValue(e.right)
         if _ival(r) is not None:
-            m = _residue(l, kn)
-            return m and (m[0], (m[1] + (r.value if e.op == '+' else -r.value)) % m[0])
+            m = _shifted(l)
+            return m and (m[0], m[1] + (r.value if e.op == '+' else -r.value))
         if e.op == '+' and _ival(l) is not None:
-            m = _residue(r, kn)
-            return m and (m[0], (m[1] + l.value) % m[0])
+            m = _shifted(r)
+            return m and (m[0], m[1] + l.value)
     return None
+
+
+def _residue(e, kn):
+    """(modulus, residue) of an expression v + c that is nowhere negative
+    (C's remainder of a negative number is negative), else None."""
+    vc = _shifted(e)
+    if vc is None or vc[0] not in kn.mod or kn.least.get(vc[0], -vc[1] - 1) + vc[1] < 0:
+        return None
+    m, r = kn.mod[vc[0]]
+    return m, (r + vc[1]) % m
 
 
 def fold(e, kn):
@@ -294,8 +316,9 @@ def fold_cond(c, kn):
     return Condition(fold(c.lhs, kn), c.conditional, fold(c.rhs, kn))
 
 
-def _mods(e, cvars):
-    """[(dimension, modulus)] of the remainders of one variable in e."""
+def _mods(e, cvars, least):
+    """[(dimension, modulus)] of the remainders in e that ``fold`` can know
+    (``least``: ``least_values``)."""
     out = []
     stack = [e]
     while stack:
@@ -305,9 +328,9 @@ def _mods(e, cvars):
             continue
         if isinstance(x, AbstractBinaryOpNode) and x.op == '%':
             m = _ival(Value.numericToValue(x.right))
-            vs = [v for v in cvars if v in x.left.collect(Variable)] if hasattr(x.left, 'collect') else []
-            if m and len(vs) == 1 and not x.left.has(Reference):
-                out.append((cvars.index(vs[0]), m))
+            vc = _shifted(x.left)
+            if m and vc and vc[0] in cvars and least.get(vc[0], -vc[1] - 1) + vc[1] >= 0:
+                out.append((cvars.index(vc[0]), m))
         if isinstance(x, Select):
             stack += [x.condition, x.true_expression, x.false_expression]
         elif isinstance(x, Reference):
@@ -681,7 +704,7 @@ class BoxPlan(GroupPlan):
             for t in stages:
                 nops += sum(_nops(p.expr) for p in t.parts) / float(len(t.parts))
                 for part in t.parts:
-                    for (k, x) in _mods(part.expr, t.func.variables):
+                    for (k, x) in _mods(part.expr, t.func.variables, least_values(t.func, part)):
                         if x in (2, 4):
                             req[k] = max(req[k], x)
         cd, rd = nd - 1, nd - 2
