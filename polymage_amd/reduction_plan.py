@@ -412,6 +412,14 @@ def _vars_of(e):
     return e.collect(Variable) if hasattr(e, 'collect') else []
 
 
+def _cond_dims(plan, rc):
+    """Dimensions of the function's own variables in a case's condition."""
+    if rc.cond is None:
+        return []
+    used = rc.cond.collect(Variable)
+    return [d for d, v in enumerate(plan.fvars) if v not in plan.rvars and any(v is u for u in used)]
+
+
 def _prod_int(xs):
     n = 1
     for x in xs:
@@ -477,18 +485,11 @@ def emit_reduction_kernel(pipe, plan, kname, mode):
             red = rc.red
             tgt = red.accumulate_ref.arguments
             w('{', ind)
-            pro = []
-            tnames = []
-            for d in range(nd):
-                q = pr.expr(tgt[d], pro)
-                if classify_access(tgt[d], plan.rvars).kind == '*':
-                    q = 'pmx_clampi(%s, %s, %s)' % (q, lbs[d], base.expr(f.domain[d].upperBound))
-                tnames.append(q)
-            val = pr.expr(red.expression, pro)
-            for l in pro:
-                w(l, ind + 1)
-            for d in range(nd):
-                w('const int q%d = %s;' % (d, tnames[d]), ind + 1)
+            # a Case's condition guards the reads of its value and of its
+            # target; only the coordinates it is on come before it
+            first = _cond_dims(plan, rc)
+            for d in first:
+                target(pr, tgt, d, ind + 1)
             conds = []
             if rc.cond is not None:
                 vn = dict(zip(plan.rvars, rnames))
@@ -500,7 +501,14 @@ def emit_reduction_kernel(pipe, plan, kname, mode):
                 cc = cpr.cond(rc.cond, cpro)
                 for l in cpro:
                     w(l, ind + 1)
-                conds.append(cc)
+                w('if (%s) {' % cc, ind + 1)
+            for d in range(nd):
+                if d not in first:
+                    target(pr, tgt, d, ind + 1)
+            pro = []
+            val = pr.expr(red.expression, pro)
+            for l in pro:
+                w(l, ind + 1)
             extra = target_ok()
             if extra:
                 conds.append(extra)
@@ -518,7 +526,16 @@ def emit_reduction_kernel(pipe, plan, kname, mode):
                 else:
                     upd = '%s = ((%s > %s)? (%s)(%s): %s);' % (slot, val, slot, T, val, slot)
             w('if (%s) { %s }' % (' && '.join(conds) or 'true', upd), ind + 1)
-            w('}', ind)
+            w('}' if rc.cond is None else '} }', ind)
+
+    def target(pr, tgt, d, ind):
+        """q<d>: the target's coordinate of dimension d."""
+        pro = []
+        q = pr.expr(tgt[d], pro)
+        if classify_access(tgt[d], plan.rvars).kind == '*':
+            q = 'pmx_clampi(%s, %s, %s)' % (q, lbs[d], base.expr(f.domain[d].upperBound))
+        for l in pro + ['const int q%d = %s;' % (d, q)]:
+            w(l, ind)
 
     def preimage():
         """lo<j>/hi<j>: the cell's points along every reduction variable."""
