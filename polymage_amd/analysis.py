@@ -593,3 +593,29 @@ def unconditional_refs(expr):
             walk(c.rhs)
     walk(expr)
     return out
+
+
+def always_refs(expr):
+    """unconditional_refs without those behind a short-circuit (the right
+    sides of && and || in a Select's condition): the reads that run at every
+    point expr is evaluated at."""
+    out = []
+
+    def walk(e):
+        e = Value.numericToValue(e)
+        if isinstance(e, Reference):
+            out.append(e)
+        if isinstance(e, Select):
+            c = e.condition
+            while c.conditional in ('&&', '||'):
+                c = c.lhs
+            walk(c.lhs)
+            walk(c.rhs)
+        elif isinstance(e, Reference):
+            for a in e.arguments:
+                walk(a)
+        elif hasattr(e, 'children'):
+            for ch in e.children():
+                walk(ch)
+    walk(expr)
+    return out

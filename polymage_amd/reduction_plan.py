@@ -30,7 +30,7 @@
 
 from fractions import Fraction
 
-from .analysis import PlanError, classify_access, case_parts, ceval_int, eval_bexpr, interval_image
+from .analysis import PlanError, always_refs, classify_access, case_parts, ceval_int, eval_bexpr, interval_image
 from .constructs import Reference, Image, Case, Reduce, Op, Reduction, Parameter
 from .cprint import Printer, c_type
 from .expr_ast import Variable, Value
@@ -420,6 +420,25 @@ def _cond_dims(plan, rc):
     return [d for d, v in enumerate(plan.fvars) if v not in plan.rvars and any(v is u for u in used)]
 
 
+def _decided(plan, rc):
+    """True, False or None (not known) for a case's condition when it is on
+    nothing but the function's dimensions that the case targets at
+    constants; True without a condition."""
+    from .box_plan import Known, decide
+    if rc.cond is None:
+        return True
+    value = {}
+    for d in _cond_dims(plan, rc):
+        try:
+            value[plan.fvars[d]] = ceval_int(rc.red.accumulate_ref.arguments[d], {})
+        except PlanError:
+            return None
+    try:
+        return decide(rc.cond, Known(value, {}))
+    except PlanError:
+        return None
+
+
 def _prod_int(xs):
     n = 1
     for x in xs:
@@ -747,9 +766,11 @@ def _emit_binned(pipe, plan, kname, mode, params, reads, buffers, exts, lbs, bas
     import itertools
     planes = list(itertools.product(*[range(lo[d], lo[d] + ext[d]) for d in others]))
     dflt = Value.numericToValue(f.default)
+    known = dict((rc, _decided(plan, rc)) for rc in plan.cases)
+    cases = [rc for rc in plan.cases if known[rc] is not False]
 
     def hits(pl):
-        return [rc for rc in plan.cases if tuple(
+        return [rc for rc in cases if tuple(
             ceval_int(rc.red.accumulate_ref.arguments[d], {}) for d in others) == pl]
 
     def counted(pl):
@@ -782,11 +803,14 @@ def _emit_binned(pipe, plan, kname, mode, params, reads, buffers, exts, lbs, bas
     f0s = [plan.floor_start(rv, plan.cases[0].red.accumulate_ref.arguments[plan.owned[rv]],
                             f.reductionDomain[j].lowerBound) for j, rv in enumerate(plan.rvars)]
 
-    # the reads of one point at affine indices
+    # the reads of one point at affine indices that run at every point: what
+    # a Case or a Select guards may lie outside its array elsewhere
     early = []
-    for rc in plan.cases:
+    for rc in cases:
+        if known[rc] is None:
+            continue
         for e in [rc.red.expression] + list(rc.red.accumulate_ref.arguments):
-            for r in (e.collect(Reference) if hasattr(e, 'collect') else []):
+            for r in always_refs(e):
                 if r.objectRef is not f and not any(a.has(Reference) for a in r.arguments if hasattr(a, 'has')):
                     text = cb(r, Printer(dict(zip(plan.rvars, rnames)), cb, mode, lazy=True), [])
                     if text not in [t for (t, _) in early]:
@@ -822,27 +846,27 @@ def _emit_binned(pipe, plan, kname, mode, params, reads, buffers, exts, lbs, bas
             text = cb(ref, pr_, pro_)
             return (regs or {}).get(text, text)
         pr = Printer(dict(zip(plan.rvars, rnames)), rcb, mode, lazy=True)
-        for rc in plan.cases:
+        for rc in cases:
             tgt = rc.red.accumulate_ref.arguments
             pl = tuple(ceval_int(tgt[d], {}) for d in others)
             if pl not in planes:
                 continue        # outside the grid
             i = planes.index(pl)
             w('{', ind)
-            pro = []
-            for d in range(nd):
+
+            def target(d):
+                pro = []
                 q = pr.expr(tgt[d], pro)
                 if classify_access(tgt[d], plan.rvars).kind == '*':
                     q = 'pmx_clampi(%s, %s, %s)' % (q, lbs[d], base.expr(f.domain[d].upperBound))
-                pro.append('const int q%d = %s;' % (d, q))
-            n = counted(pl)
-            if n is None:
-                val = pr.expr(rc.red.expression, pro)
-                pro.append('const auto pmx_v = %s;' % val)
-            for l in pro:
-                w(l, ind + 1)
+                for l in pro:
+                    w(l, ind + 1)
+                return q
             conds = []
-            if rc.cond is not None:
+            first = [] if known[rc] else _cond_dims(plan, rc)
+            for d in first + ([d for d in od if d not in first] if owned else []):
+                w('const int q%d = %s;' % (d, target(d)), ind + 1)
+            if not known[rc]:
                 vn = dict(zip(plan.rvars, rnames))
                 for v, d in zip(plan.fvars, range(nd)):
                     if v not in plan.rvars:
@@ -855,8 +879,19 @@ def _emit_binned(pipe, plan, kname, mode, params, reads, buffers, exts, lbs, bas
                 conds += ['q%d == c%d' % (d, d) for d in od]
             if inside:
                 conds.append(inside)
+            if conds:
+                w('const bool pmx_c = %s;' % ' && '.join(conds), ind + 1)
+            # a condition guards the reads of the bin and of the value
+            n = counted(pl)
+            q = 'q%d' % z if z in first else target(z)
             w('const int pmx_z = %s - (%d) - pmx_h;' % (
-                '((%s) ? q%d : %d)' % (' && '.join(conds), z, lo[z] - 2 * G) if conds else 'q%d' % z, lo[z]), ind + 1)
+                '(pmx_c ? %s : %d)' % (q, lo[z] - 2 * G) if conds else q, lo[z]), ind + 1)
+            if n is None:
+                pro = []
+                val = pr.expr(rc.red.expression, pro)
+                for l in pro:
+                    w(l, ind + 1)
+                w('const auto pmx_v = %s;' % (val if known[rc] else 'pmx_c ? (%s) : 0' % val), ind + 1)
             op = rc.red.op_type
             s = 'a%d[g]' % i
             upd = '%s += 1' % s if n is not None else \

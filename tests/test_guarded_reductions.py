@@ -71,7 +71,7 @@ BINNED = ['value', 'select', 'and', 'or', 'bin', 'plane']
 SIZES = [(32, 64), (33, 70)]
 
 
-def _check(form, R, C, opts, gpu=False):
+def _check(form, R, C, opts):
     g, pipe, vals, shape, typ = _case(form, R, C, opts)
     plan = plan_pipeline(pipe)[0]
     assert (plan.owner and plan.bin_dim is not None) == (form != 'atomic' and not opts)
@@ -98,3 +98,18 @@ def _under_asan(forms, opts):
 @pytest.mark.parametrize("form", BINNED + ['atomic'])
 def test_guarded_reads_under_asan(form):
     _under_asan([form], {'no_bins': 1} if form != 'atomic' else None)
+
+
+def test_binned_guarded_reads_under_asan():
+    _under_asan(BINNED, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("opts", [None, {'no_bins': 1}])
+@pytest.mark.parametrize("form", BINNED + ['atomic'])
+def test_guarded_reductions_bitexact(gpu, form, opts):
+    if emulating():
+        pytest.skip("covered by the emulator tests")
+    for R, C in SIZES:
+        print("case guarded", form, R, C, opts, flush=True)
+        _check(form, R, C, opts)
