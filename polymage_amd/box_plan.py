@@ -679,8 +679,9 @@ class BoxPlan(GroupPlan):
         Constant dimensions of up to 8 points are taken whole when points
         along them share reads (colours that all read alpha, intensity
         levels of one gray value) or differ in their Case; along rows and
-        columns the block is a multiple of every parity (period up to 4)
-        that an index or remainder of the stage uses.  Among the sizes left,
+        columns the block is a multiple of every parity (period 2 or 4)
+        that an index or remainder of the stage uses; an index of another
+        period is computed per point.  Among the sizes left,
         the smallest of an estimate is taken: (wavefronts of items, half of
         them rounded up to whole workgroup iterations) x (fixed cost + points
         x operations + distinct loads)."""
@@ -699,7 +700,7 @@ class BoxPlan(GroupPlan):
                 ms = [arg_map(x, t.func.variables) for x in r.arguments]
                 maps.append((t, r, ms))
                 for x in ms:
-                    if x.kind == 'var' and 1 < x.period <= 4:
+                    if x.kind == 'var' and x.period in (2, 4):
                         req[x.dim] = max(req[x.dim], x.period)
             for t in stages:
                 nops += sum(_nops(p.expr) for p in t.parts) / float(len(t.parts))
@@ -758,6 +759,8 @@ class BoxPlan(GroupPlan):
                 waves = 0.5 * (-(-items // 64)) + 0.5 * (-(-items // threads)) * (threads / 64.0)
                 if best is None or (waves * c, -pts) < best[0]:
                     best = ((waves * c, -pts), b)
+        if best is None:
+            raise PlanError("no block holds every parity of %s" % s.name)
         for m in members:
             m.blk = list(best[1])
             m.base = [sp.lo for sp in span]
