@@ -303,11 +303,19 @@ def fold(e, kn):
                 if te is not tt:
                     x = Cast(tt, x)
             return x
-        return Select(fold_cond(e.condition, kn), fold(e.true_expression, kn),
-                      fold(e.false_expression, kn), False)
+        return Select(fold_cond(e.condition, kn), _typed(fold(e.true_expression, kn), e.true_expression),
+                      _typed(fold(e.false_expression, kn), e.false_expression), False)
     if isinstance(e, InbuiltFunction):
         return type(e)(*[fold(a, kn) for a in e.arguments])
     raise PlanError("cannot fold %s" % (e,))
+
+
+def _typed(x, e):
+    """x, folded from a select's branch e, with e's DSL type (a folded
+    constant is an Int whatever its parts' types; a select's branches have
+    one type)."""
+    t = getType(Value.numericToValue(e))
+    return x if getType(x) is t else Cast(t, x)
 
 
 def fold_cond(c, kn):
