@@ -279,8 +279,9 @@ def fold(e, kn):
         l, r = fold(e.left, kn), fold(e.right, kn)
         if _ival(l) is not None and _ival(r) is not None and e.op in ('+', '-', '*', '/', '%') and \
                 not (e.op in '/%' and r.value == 0):
+            # (a literal outside int makes C's arithmetic long long)
             v = ceval_int(_rebuild_bin(e, l, r), {})
-            if -2 ** 31 <= v < 2 ** 31:
+            if all(-2 ** 31 <= i < 2 ** 31 for i in (v, l.value, r.value)):
                 return Value(v, Int)
         return _rebuild_bin(e, l, r)
     if isinstance(e, AbstractUnaryOpNode):

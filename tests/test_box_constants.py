@@ -1,5 +1,5 @@
 """Constants that box kernels fold: selects with a branch of typed integer
-constants, and planes whose variable is not an Int, against the general
+constants, literals that C holds in a long, and planes whose variable is not an Int, against the general
 kernels' path and the oracle."""
 import numpy as np
 import pytest
@@ -28,13 +28,16 @@ def _case(form, opts=None):
     bright = Condition(img(x, y), '>', 0.5)
     out.defn = [{'minus': lambda: Select(bright, -Value(1, Float), a(x - 1, y + 1)),
                  'sum': lambda: Select(bright, a(x - 1, y + 1), Value(1, Float) + Value(2, Float)),
+                 # (an int would overflow)
+                 'long': lambda: a(x - 1, y) + Cast(Float, (Value(2 ** 31 + 5, Int) - Value(2 ** 31, Int)) *
+                                                   (x * 40000000)),
                  'plane': lambda: a(x - 1, y) + Select(Condition(x, '>', 7), c, Value(3, UInt))}[form]()]
     pipe = build(out, {'R': R, 'C': C}, {'R': 96, 'C': 144}, 'boxconst_' + form, [16, 32], gpu_options=opts)
     img_ = np.random.default_rng(3).random((N, M)).astype(np.float32)
     return out, pipe, {'R': N, 'C': M, 'img': img_}, shape
 
 
-FORMS = ['minus', 'sum', 'plane']
+FORMS = ['minus', 'sum', 'long', 'plane']
 
 
 def _check(out, run, vals, shape):
