@@ -718,8 +718,11 @@ def _stores(B, item, m, mi, pts, SL):
             for i, b in coef:
                 terms.append('(unsigned)j%d * %s' % (i, '(unsigned)(S_%s_%d * %d)' % (f.name, i, b)
                                                      if i < m.nd - 1 else '%du' % b))
-            return 'const unsigned %s = (%s) * %du;' % (n, ' + '.join(terms) or '0u', f.typ.nbytes())
-        return 'pmx_at(%s, %s)' % (B.uni[key], item.base(okey, mk))
+            e = ' + '.join(terms) or '0u'
+            return 'const unsigned %s = %s;' % (n, e if B.edge else '(%s) * %du' % (e, f.typ.nbytes()))
+        # (the edge version serves every tile of an array above 4 GiB: its
+        # offsets count elements, of which an array has fewer than 2^31)
+        return ('(%s + %s)' if B.edge else 'pmx_at(%s, %s)') % (B.uni[key], item.base(okey, mk))
 
     # points of a block that the box does not hold (its extent is no whole
     # number of blocks, or the block grid starts before it)
