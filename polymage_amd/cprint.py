@@ -523,18 +523,19 @@ __device__ __forceinline__ int pmx_find_frame(const long long* first, const int 
   while (lo < hi) { const int mid = (lo + hi + 1) >> 1; if (first[mid] <= t) lo = mid; else hi = mid - 1; }
   return lo;
 }
-// the same for wavefronts of 64 active lanes, 64 frames per step, one a lane
-// (a search by halves is a chain of six dependent loads for 48 frames)
+// the same for wavefronts of 64 active lanes: a 64-way search, one entry a
+// lane, so 64 frames take one step and 4096 two (a search by halves is a
+// chain of six dependent loads for 48 frames)
 __device__ __forceinline__ int pmx_find_frame64(const long long* first, const int n, const long long t) {
 #ifdef PMX_DEVICE_AS
-  int c = 0;
-  for (int b = 0; b < n; b += 64) {
-    const int i = b + (int)(threadIdx.x & 63u);
-    const int k = __popcll(__ballot(i < n && first[i < n ? i : 0] <= t));
-    c += k;
-    if (k < 64) break;
+  int lo = 0, step = 1;
+  while (step < (n + 63) / 64) step *= 64;
+  for (;; step /= 64) {
+    const int i = lo + (int)(threadIdx.x & 63u) * step;
+    lo += (__popcll(__ballot(i < n && first[i < n ? i : 0] <= t)) - 1) * step;
+    if (step == 1) break;
   }
-  return __builtin_amdgcn_readfirstlane(c - 1);
+  return __builtin_amdgcn_readfirstlane(lo);
 #else
   return pmx_find_frame(first, n, t);
 #endif
