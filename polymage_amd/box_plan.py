@@ -47,6 +47,11 @@ GENERAL_ONLY = ('block', 'block_lds', 'lanes', 'stage', 'no_inline', 'no_fuse', 
 MAX_POINTS = 16         # points of one per-thread block (registers)
 
 
+def resident(threads, lds):
+    """Workgroups a compute unit holds, by threads and bytes of LDS."""
+    return min(2048 // threads, (160 * 1024) // max(1, lds))
+
+
 def _has_param(e):
     return any(isinstance(v, Parameter) for v in e.collect(Variable)) if hasattr(e, 'collect') else False
 
@@ -392,8 +397,28 @@ class BoxPlan(GroupPlan):
         o = plan.opts
         if o.get('no_box') or any(o.get(k) for k in GENERAL_ONLY) or int(o.get('roll', 1)) > 1:
             return None
+        def boxes(**opts):
+            return BoxPlan(plan.pipe, plan.group, plan.gindex, plan.tile_sizes, dict(o, **opts))
         try:
-            return BoxPlan(plan.pipe, plan.group, plan.gindex, plan.tile_sizes, plan.opts)
+            box = boxes()
+            # LDS rows hold whole blocks, and the rows that pads cost can
+            # halve the workgroups a compute unit holds: blocks of fewer rows
+            # then, if they bring those back.  Harris, 16x512 tiles of 512
+            # threads, 82.6 KB of LDS against 74.3 (general 74.3), us at
+            # 1200x1600 / 2048x2048 / 3000x3000 / 4100x4100: 16.1 / 16.6 /
+            # 31.3 / 55.6 with 4x2 blocks, 14.4 / 15.4 / 27.7 / 43.5 with
+            # 2x2, general kernel 13.2 / 14.6 / 32.2 / 56.9.  (Two workgroups
+            # instead of three are no reason: 16x340, w256, 11.9 / 18.9 / 31.9
+            # / 51.5 against 12.6 / 19.1 / 29.9 / 47.9.)
+            threads = int(o.get('threads', 256))
+            want = resident(threads, plan.lds_bytes)
+            for rows in (2, 1):
+                if 2 * resident(threads, box.lds_bytes) > want:
+                    break
+                less = boxes(box_rows=rows)
+                if resident(threads, less.lds_bytes) >= want:
+                    box = less
+            return box
         except PlanError:
             return None
 
@@ -747,6 +772,9 @@ class BoxPlan(GroupPlan):
         for U in ((1, 2, 4, 8) if rd >= 0 and best is None else (1,) if best is None else ()):
             for V in (1, 2, 4):
                 if rd >= 0 and U % req[rd] or V % req[cd]:
+                    continue
+                if rd >= 0 and U > max(int(self.opts.get('box_rows', U)), req[rd]) and \
+                        any(m.needs_lds for m in members):
                     continue
                 least = (req[rd] if rd >= 0 else 1) * req[cd]
                 if U * V > least and (whole * U * V > MAX_POINTS or

@@ -27,7 +27,7 @@ from .analysis import PlanError, classify_access, eval_bexpr, unconditional_refs
 from .constructs import Reference, Image, Case, Reduction
 from .cprint import Printer, DEVICE_PRELUDE, c_type
 from .box_emit import BOX_PRELUDE, emit_box_kernel
-from .box_plan import BoxPlan
+from .box_plan import BoxPlan, resident
 from .group_plan import GroupPlan
 from .region_ir import REGION_PRELUDE, bound_c
 from .reduction_plan import ReductionPlan, emit_reduction_kernel, ConstPlan, emit_const_kernel
@@ -1312,10 +1312,6 @@ def _levels(kernels):
     return [[k for k, l in zip(kernels, level) if l == n] for n in range(max(level + [-1]) + 1)]
 
 
-def _resident(k, lds):
-    return min(2048 // k.threads, (160 * 1024) // max(1, lds))
-
-
 def plan_launches(pipe, kernels, params):
     """(source of the plain entry points, launches in order).
 
@@ -1338,7 +1334,7 @@ def plan_launches(pipe, kernels, params):
                 group += same
                 group.sort(key=lambda x: -x.work)
                 lds = max(x.lds for x in group)
-                if _resident(group[0], lds) < _resident(group[0], group[0].lds):
+                if resident(k.threads, lds) < resident(k.threads, group[0].lds):
                     group = [k]
             rest = [x for x in rest if x not in group]
             if len(group) == 1:
