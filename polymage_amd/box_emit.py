@@ -310,7 +310,10 @@ class _Item(object):
             fast = 'pmx_at(%s, %s)[%d]' % (B.uni[key], ' + '.join([off] + dyn), c)
             if not B.edge:
                 return fast
-            ekey = (key, okey, c)
+            # (reads of one element that are clamped differently differ in
+            # their clamped form)
+            ekey = (key, okey, c, tuple((tuple(B.bound(b) for b in m.lows), tuple(B.bound(b) for b in m.highs))
+                                        for m in maps))
             if ekey not in self.early:
                 reg = 'ge%d' % len(self.early)
                 self.early[ekey] = (reg, c_type(f.typ), fast, self.clamped(f, ref, t))
