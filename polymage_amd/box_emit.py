@@ -712,7 +712,9 @@ def _stores(B, item, m, mi, pts, SL):
                 terms.append('(%s - LB_%s_%d)%s' % (B.coord(s.span[i], c), f.name, i,
                                                     ' * S_%s_%d' % (f.name, i) if i < m.nd - 1 else ''))
             B.uni[key] = g
-            B.uni_lines.append('const auto %s = G_%s + (%s);' % (g, f.name, ' + '.join(terms) or '0'))
+            e = ' + '.join(terms) or '0'
+            B.uni_lines.append('const int %s = %s;' % (g, e) if B.edge else
+                               'const auto %s = G_%s + (%s);' % (g, f.name, e))
         coef = tuple((i, s.blk[i]) for i in range(m.nd) if s.cnt[i] > 1)
         okey = ('gs', f.name)
 
@@ -725,7 +727,8 @@ def _stores(B, item, m, mi, pts, SL):
             return 'const unsigned %s = %s;' % (n, e if B.edge else '(%s) * %du' % (e, f.typ.nbytes()))
         # (the edge version serves every tile of an array above 4 GiB: its
         # offsets count elements, of which an array has fewer than 2^31)
-        return ('(%s + %s)' if B.edge else 'pmx_at(%s, %s)') % (B.uni[key], item.base(okey, mk))
+        off = item.base(okey, mk)
+        return '(G_%s + (%s + %s))' % (f.name, off, B.uni[key]) if B.edge else 'pmx_at(%s, %s)' % (B.uni[key], off)
 
     # points of a block that the box does not hold (its extent is no whole
     # number of blocks, or the block grid starts before it)
