@@ -339,7 +339,7 @@ class ReductionPlan(object):
         owner-cell reduction whose other free dimensions every case targets
         at constants and whose cells have constant pre-images: its cells'
         accumulators then fit in registers (_emit_binned).  None if there is
-        no such dimension."""
+        no such dimension, or accumulators in LDS are faster."""
         f = self.func
         ks = [self.pre_size.get(rv) for rv in self.rvars]
         if not all(ks) or _prod_int(ks) > 256:
@@ -367,7 +367,26 @@ class ReductionPlan(object):
         half = (ext[z] + 1) // 2
         if len(consts) != len(self.cases) or ext[z] < 2 or half * other > self.MAX_BINS:
             return None
-        return z
+        # Against LDS accumulators, times of LDS / registers at 300 x 400,
+        # 1083 x 1923 and 2560 x 1536 (whose cells are all whole):
+        # every bin costs a thread a compare and an update per point, more
+        # than one LDS update beyond 8 bins: 32 bins on 8 x 8 cells 0.93 0.87
+        # 0.58, 16 bins 1.44 1.21 0.79, 8 bins 2.01 1.55 1.00;
+        # cells of few points have wavefronts enough to hide the LDS, unless
+        # it holds many accumulators: 2 x 2 cells, 8 bins 0.98 0.94 0.93, 12
+        # bins 0.99 1.20 1.23; 4 x 2 cells, 6 bins 0.96 1.02 0.81; 4 x 4, 8
+        # bins 1.00 1.32 0.76; 8 x 4, 4 bins 1.93 2.18 0.91;
+        # a Case decided at run time keeps its reads behind it, so that they
+        # no longer issue together: 8 x 8 cells, two planes of 14 bins 0.54
+        # 0.62 1.13, of 4 bins 0.58 0.60 1.03 - only small cells with more
+        # accumulators than the LDS kernel holds well gain then: 4 x 4 cells,
+        # two planes of 8 bins 0.96 0.75 0.75, of 10 bins 1.15 1.18 1.56.
+        points, acc = _prod_int(ks), ext[z] * other
+        if half > 8:
+            return None
+        if any(_decided(self, rc) is None for rc in self.cases):
+            return z if points <= 16 and other > 1 and acc > 16 else None
+        return z if points >= 8 or acc >= 12 else None
 
     def floor_start(self, rv, arg, lower):
         """f0 when ``arg`` is f0 + rv / k for every rv >= 0 the domain holds

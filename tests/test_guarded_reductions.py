@@ -35,10 +35,19 @@ def _case(form, R, C, opts=None):
                       dom, Float, 'grid')
         at, shape = (lambda e: g(x / 4, y / 4, b(e))), (R // 4 + 1, C // 4 + 1, 6)
     inner, last = Condition(x, '>=', 1), Condition(x, '<', rows - 1)
+    if form in ('value', 'bin', 'plane'):
+        # planes decided by their constant index, with and without a guard
+        # too (the kernel with bins in registers serves guarded cases of more
+        # than 16 accumulators)
+        g = Reduction(([c, x, y, z], [Interval(Int, 0, 1), Interval(Int, 0, rows / 4), Interval(Int, 0, cols / 4),
+                                      Interval(Int, 0, 9)]), dom, Float, 'grid')
+        at, shape = (lambda k, e: g(k, x / 4, y / 4, b(e))), (2, R // 4 + 1, C // 4 + 1, 10)
     if form == 'value':
-        g.defn = [Case(inner, Reduce(at(img(x, y)), img(x, y) - img(x - 1, y), Op.Sum))]
+        g.defn = [Case(inner, Reduce(at(0, img(x, y)), img(x, y) - img(x - 1, y), Op.Sum)),
+                  Case(last, Reduce(at(1, img(x, y)), img(x, y) * img(x + 1, y), Op.Max))]
     elif form == 'select':
-        g.defn = [Case(inner, Reduce(at(img(x, y)), img(x - 1, y) + Select(last, img(x + 1, y), img(x, y)), Op.Sum))]
+        g.defn = [Reduce(at(img(x, y)), Select(inner, img(x - 1, y), img(x, y)) + Select(last, img(x + 1, y), img(x, y)),
+                         Op.Sum)]
     elif form == 'and':
         # the right side of && reads only where the left one holds
         g.defn = [Reduce(at(img(x, y)), Select(inner & Condition(img(x - 1, y), '>', 0.5), img(x, y), img(x, y) * 2.0),
@@ -47,16 +56,12 @@ def _case(form, R, C, opts=None):
         g.defn = [Reduce(at(img(x, y)), img(x, y) * Select(Condition(x, '<', 1) | Condition(img(x - 1, y), '>', 0.5),
                                                           img(x, y), img(x, y) + 2.0), Op.Sum)]
     elif form == 'bin':
-        g.defn = [Case(inner, Reduce(at(img(x - 1, y)), img(x, y), Op.Sum)),
-                  Case(Condition(x, '<', 1), Reduce(at(img(x, y)), img(x + 1, y), Op.Sum))]
+        g.defn = [Case(inner, Reduce(at(0, img(x - 1, y)), img(x, y), Op.Sum)),
+                  Case(Condition(x, '<', 1), Reduce(at(1, img(x, y)), img(x + 1, y), Op.Sum))]
     elif form == 'plane':
-        # planes decided by their constant index, one of them guarded too
-        g = Reduction(([c, x, y, z], [Interval(Int, 0, 1), Interval(Int, 0, rows / 4), Interval(Int, 0, cols / 4),
-                                      Interval(Int, 0, 5)]), dom, Float, 'grid')
-        g.defn = [Case(Condition(c, '==', 0) & inner, Reduce(g(0, x / 4, y / 4, b(img(x, y))), img(x - 1, y), Op.Sum)),
-                  Case(Condition(c, '==', 1), Reduce(g(1, x / 4, y / 4, b(img(x, y))), 1, Op.Sum)),
-                  Case(Condition(c, '==', 0), Reduce(g(1, x / 4, y / 4, b(img(x, y))), 5, Op.Sum))]
-        shape = (2,) + shape
+        g.defn = [Case(Condition(c, '==', 0) & inner, Reduce(at(0, img(x, y)), img(x - 1, y), Op.Sum)),
+                  Case(Condition(c, '==', 1), Reduce(at(1, img(x, y)), 1, Op.Sum)),
+                  Case(Condition(c, '==', 0), Reduce(at(1, img(x, y)), 5, Op.Sum))]
     else:
         g.defn = [Case(inner, Reduce(at(img(x - 1, y)), Cast(Int, img(x - 1, y) * 100), Op.Sum))]
     g.default = 0
@@ -102,6 +107,24 @@ def test_guarded_reads_under_asan(form):
 
 def test_binned_guarded_reads_under_asan():
     _under_asan(BINNED, None)
+
+
+@pytest.mark.parametrize("cell,bins,planes,guard,binned", [
+    ((8, 8), 14, 2, False, True), ((8, 8), 8, 1, False, True), ((8, 8), 32, 1, False, False),
+    ((2, 2), 8, 1, False, False), ((2, 2), 12, 1, False, True), ((4, 2), 6, 1, False, True),
+    ((8, 8), 14, 2, True, False), ((4, 4), 8, 2, True, False), ((4, 4), 10, 2, True, True)])
+def test_where_bins_go_to_registers(cell, bins, planes, guard, binned):
+    rows, cols = Parameter(Int, 'rows'), Parameter(Int, 'cols')
+    x, y, z, c = (Variable(Int, n) for n in 'xyzc')
+    img = Image(Float, 'img', [rows, cols])
+    g = Reduction(([c, x, y, z], [Interval(Int, 0, planes - 1), Interval(Int, 0, rows / cell[0]),
+                                  Interval(Int, 0, cols / cell[1]), Interval(Int, 0, bins - 1)]),
+                  ([x, y], [Interval(Int, 0, rows - 1), Interval(Int, 0, cols - 1)]), Float, 'grid')
+    red = [Reduce(g(k, x / cell[0], y / cell[1], Cast(Int, img(x, y) * 3)), img(x, y), Op.Sum) for k in range(planes)]
+    g.defn = [Case(Condition(x, '>=', 1), r) if guard else r for r in red]
+    g.default = 0
+    pipe = build(g, {'rows': rows, 'cols': cols}, {'rows': 64, 'cols': 64}, 'where_bins', [16, 16])
+    assert (plan_pipeline(pipe)[0].bin_dim is not None) == binned
 
 
 @pytest.mark.gpu
