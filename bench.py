@@ -433,7 +433,10 @@ def app_entry(args, torch, dev, app, cpu, headline=None):
     else:
         ent['exhaustive'] = 'same schedule as learned'
         r1 = r0
-    ent['learned_over_exhaustive_mpix'] = round(r1['ms_per_call'] / r0['ms_per_call'], 4)
+    # (the exhaustive pick is a search's; the learned one gives way to a sweep
+    # over several sizes where one is recorded, and is no search's result then)
+    kind = 'swept' if r0['schedule'].startswith('swept') else 'learned'
+    ent[kind + '_over_exhaustive_mpix'] = round(r1['ms_per_call'] / r0['ms_per_call'], 4)
     ent['recorded_tuning'] = recorded_tuning(app)
     ent['ideal_bytes'] = w0.ideal_bytes
     ent['mpix'] = round(w0.mpix, 4)
@@ -447,9 +450,9 @@ def app_entry(args, torch, dev, app, cpu, headline=None):
 
 def classed_batch(args, torch, w, recs, outs, refs, stream):
     """The same frames split into the autotuner's size classes, each class
-    through its own compiled pipeline (the tiles tuned on a persistent
-    launch over that class's frames): one persistent launch per class, each
-    on a stream of its own so they overlap, and the classes' captured
+    through its own compiled pipeline (the tiles tuned on a batch launch
+    of the general kernels over that class's frames): one launch per class,
+    each on a stream of its own so they overlap, and the classes' captured
     graphs likewise.  Every frame is compared with the oracle after each
     mode.  None when no classes are recorded."""
     import numpy as np
@@ -467,8 +470,8 @@ def classed_batch(args, torch, w, recs, outs, refs, stream):
     classes = [{'max_area': a} for (a, _, _, _, _) in sched]
     cb = ClassedBatch(built, classes, recs, lambda r: r['R'] * r['C'])
     # one side stream per class (default priority), ordered after the
-    # timing stream and joined back into it, so the classes' persistent
-    # launches overlap each other's tails
+    # timing stream and joined back into it, so the classes' launches
+    # overlap each other's tails
     main = torch.cuda.current_stream()
     side = [torch.cuda.Stream() for _ in sched]
 
@@ -513,7 +516,7 @@ def classed_batch(args, torch, w, recs, outs, refs, stream):
 
 def batch_entry(args, torch, dev, cpu):
     """48 camera-pipeline frames of uneven sizes (uint16 Bayer in, uint8 RGB
-    out): one persistent work-queue launch per kernel over all frames, the
+    out): one launch per kernel over the work items of all frames, the
     same launches replayed from a hipGraph, per-frame plain launches issued
     back to back, and per-frame plain calls one at a time (each waited
     for).  Every frame of the last persistent, graph and per-frame runs is
