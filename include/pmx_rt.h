@@ -61,9 +61,11 @@ int pmx_launch(void* function, unsigned gx, unsigned gy, unsigned gz,
                void* stream, void** args);
 
 /* Resident workgroups of `function` per compute unit at `threads` threads
- * and `dyn_lds` bytes of dynamic LDS (sizes persistent launches). */
+ * and `dyn_lds` bytes of dynamic LDS.  Called, like pmx_device_cus, by
+ * pipeline libraries built while a batch ran on a resident grid of
+ * workgroups; newly generated ones launch a workgroup per work item. */
 int pmx_occupancy(void* function, int threads, size_t dyn_lds, int* blocks_per_cu);
-/* Compute units of device `dev`. */
+/* Compute units of device `dev` (see pmx_occupancy). */
 int pmx_device_cus(int dev, int* n);
 
 /* ---- streams, events, graphs --------------------------------------------- */

@@ -53,7 +53,6 @@ template <typename V, typename T> static inline V pmx_ld4(const T* p) {
 #define __builtin_amdgcn_readfirstlane(v) (v)
 #define PMX_GLOBAL
 #define PMX_CONST
-#define PMX_OPAQUE(x)
 static inline int __mul24(int a, int b) { return a * b; }
 static inline unsigned __umul24(unsigned a, unsigned b) { return a * b; }
 static inline int atomicOr(int* p, int v) { return __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }
