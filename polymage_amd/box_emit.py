@@ -224,7 +224,14 @@ class _Item(object):
                 q = pr.expr(arg, pro)
                 dyn.append('__mul24(%s - %s, %d)' % (q, self.B.coord(sp, sp.lo), W[i]))
                 continue
-            q = 'pmx_clampi(%s, %d, %d)' % (pr.expr(arg, pro), p.span[i].lo, p.span[i].hi)
+            q = pr.expr(arg, pro)
+            if sp.A:
+                # (a choice between two indices that are each as above: a
+                # data-dependent index has no constant box but a constant
+                # axis)
+                dyn.append('__mul24(%s - %s, %d)' % (q, self.B.coord(sp, sp.lo), W[i]))
+                continue
+            q = 'pmx_clampi(%s, %d, %d)' % (q, p.span[i].lo, p.span[i].hi)
             dyn.append('__mul24(%s - %s, %d)' % (q, _c(sp.lo), W[i]))
         key = ('l', tuple(sorted(coef.items())))
         nm = self.base(key, lambda n: 'const int %s = %s;' % (n, ' + '.join(

@@ -1,16 +1,18 @@
-"""Box kernels with scales that are no powers of two: thirds of an in-group
-stage and of an image, beside halves, and every third point; against the
-general kernels' path and the oracle.  Tiles that are and are not multiples
-of the scale."""
+"""Box kernels with indices computed per point: thirds of an in-group stage
+and of an image, beside halves, and every third point; selects between two
+such reads (their indices are selected, one read is left), by 3, by 8 and of
+halves in blocks that do not know the parity; against the general kernels'
+path and the oracle.  Tiles that are and are not multiples of the scale."""
 import numpy as np
 import pytest
 
 from oracle import cemit
-from polymage_amd.constructs import Parameter, Variable, Interval, Image, Function, Int, Float
+from polymage_amd.constructs import Parameter, Variable, Interval, Image, Function, Condition, Select, Int, Float
 
 from helpers import build, bits_equal, gpu_build, emulating
 
-FORMS = ['stage', 'image', 'halves', 'sixths', 'every_third']
+FORMS = ['stage', 'image', 'halves', 'sixths', 'every_third', 'select3', 'select8', 'parity']
+BOXES = ('stage', 'image', 'every_third', 'select3', 'parity')      # (an axis read at two scales has no constant box)
 
 
 def _case(form, R_, C_, tiles, opts=None):
@@ -27,7 +29,13 @@ def _case(form, R_, C_, tiles, opts=None):
                  'image': lambda: img(x / 3, y / 3) - a(x + 1, y),
                  'halves': lambda: a(x / 3, y / 2) + a(x / 2, y / 3) * img(x / 2, (y + 1) / 2),
                  'sixths': lambda: a(x / 2 / 3, (y + 1) / 3 / 2) + a(x / 4, y / 3),
+                 'select3': lambda: Select(Condition(x % 3, '==', 0), a(x / 3, y / 3), a(x / 3 + 1, y / 3)),
+                 'select8': lambda: Select(Condition(x % 8, '<', 4), a(x / 8, y / 8), a(x / 8 + 1, y / 8)),
+                 'parity': lambda: Select(Condition(x % 2, '==', 0), a(x / 2, y / 2), a(x / 2 + 1, y / 2)) +
+                 Select(Condition(y % 2, '==', 0), a(x / 2, y / 2), a(x / 2, y / 2 + 1)),
                  'every_third': lambda: a(3 * x + 1, 3 * y) + a(3 * x, 3 * y + 2)}[form]()]
+    if form == 'parity' and not (opts or {}).get('no_box'):
+        opts = dict(opts or {}, box_blocks={'out': [1, 1]})
     pipe = build(out, {'R': R, 'C': C}, {'R': 320, 'C': 440}, 'boxscale_' + form, tiles, gpu_options=opts)
     img_ = np.random.default_rng(R_).random((R_, C_)).astype(np.float32)
     return out, pipe, {'R': R_, 'C': C_, 'img': img_}, shape
@@ -52,8 +60,7 @@ def test_scales_on_the_emulator(form, R, C, tiles, opts):
     from polymage_amd.box_plan import BoxPlan
     from polymage_amd.hip_emit import plan_pipeline
     out, pipe, vals, shape = _case(form, R, C, tiles, opts)
-    if opts is None and tiles != [16, 32] and form in ('stage', 'image', 'every_third'):
-        # (an axis read at two scales has no constant box)
+    if opts is None and tiles != [16, 32] and form in BOXES:
         assert all(BoxPlan.of(p) is not None for p in plan_pipeline(pipe))
     _check(out, kernel_emu.build(pipe).run_host, vals, shape)
 
