@@ -24,7 +24,7 @@ import hashlib
 import re
 
 from .analysis import PlanError, classify_access, eval_bexpr, unconditional_refs, shift_access, scaled_access
-from .constructs import Reference, Image, Case, Reduction
+from .constructs import Reference, Image, Case, Reduction, Select
 from .cprint import Printer, DEVICE_PRELUDE, c_type
 from .box_emit import BOX_PRELUDE, emit_box_kernel
 from .box_plan import BoxPlan, resident
@@ -796,6 +796,7 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True, forms=FORMS):
                     vprobe.d = dvec(u, v)
                     emit_point([], m, vprobe, body_ind, 'x', 'y')
             vmap = {}
+            rows = []
             for n, key in enumerate(sorted(vprobe.vprobe, key=str)):
                 p, cols = vprobe.vprobe[key]
                 cmin = min(cols)
@@ -812,6 +813,24 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True, forms=FORMS):
                 for c in range(nch):
                     vloads.append('  ' * body_ind + 'const %s %s_%d = pmx_ld4<%s>(&L_%s[%s + %d]);' % (
                         vt, prefix, c, vt, p.name, idx, 4 * c))
+                rows.append((p, key, idx, cmin, nch))
+            # a row that only some of the block's Cases or Selects read may
+            # lie outside what the tile computes of its producer (a tile
+            # without border points computes nothing for the border's Case):
+            # the block's points then take their own branches
+            if any(len(t.parts) > 1 or part.expr.has(Select)
+                   for m in members for t in [m] + inline_closure(m) for part in t.parts):
+                ends = {}
+                for p, key, idx, cmin, nch in rows:
+                    W = [_prod(plan.lds_ext(p)[j + 1:]) for j in range(p.nd)]
+                    if all(isinstance(o, int) for o in key[2]):
+                        at, first = fitem.lds_base(p, key[1]), sum(o * x for o, x in zip(key[2], W)) + cmin
+                    else:
+                        at, first = '(%s)' % idx, 0
+                    lo, hi, _ = ends.get((p.name, at), (first, first, p))
+                    ends[(p.name, at)] = (min(lo, first), max(hi, first + 4 * nch), p)
+                for (_, at), (lo, hi, p) in sorted(ends.items(), key=str):
+                    vconds += ['%s >= %d' % (at, -lo), '%s <= %d' % (at, p.lds_size // p.func.typ.nbytes() - hi)]
         fast = list(vloads)
         for mi, m in enumerate(members):
             T = c_type(m.func.typ)
