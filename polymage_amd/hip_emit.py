@@ -23,9 +23,11 @@ reference, and ``pipeline_<name>_dev(..., stream)`` on device pointers.
 import hashlib
 import re
 
-from .analysis import PlanError, classify_access, eval_bexpr, unconditional_refs, shift_access, scaled_access
+from .analysis import (PlanError, always_refs, classify_access, eval_bexpr, unconditional_refs, shift_access,
+                       scaled_access)
 from .constructs import Reference, Image, Case, Reduction, Select
-from .cprint import Printer, DEVICE_PRELUDE, c_type
+from .cprint import Printer, DEVICE_PRELUDE, c_type, same_expr
+from .expression import substitute_vars
 from .box_emit import BOX_PRELUDE, emit_box_kernel
 from .box_plan import BoxPlan, resident
 from .group_plan import GroupPlan
@@ -520,6 +522,34 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True, forms=FORMS):
         visit(s)
         return out
 
+    needs = {}
+
+    def always(s):
+        """References (in s's variables) that are read at every point of s."""
+        common = None
+        for part in s.parts:
+            refs = [] if part.pred else always_refs(part.expr)
+            for r in list(refs):
+                if plan.in_group(r.objectRef) and plan.stage_of(r.objectRef).inline:
+                    t = plan.stage_of(r.objectRef)
+                    ren = dict(zip(t.func.variables, s.func.variables))
+                    refs += [substitute_vars(x, ren) for x in always(t)]
+            common = refs if common is None else [x for x in common if any(same_expr(x, r) for r in refs)]
+        return common or []
+
+    def conditional(s, t):
+        """True when inlined stage t reads what points of s may do without
+        (only some of its Cases or a Select's branch use t): t is then
+        evaluated inside its region only, outside it its reads may leave
+        their arrays."""
+        known = always(s)
+        ren = dict(zip(t.func.variables, s.func.variables))
+        if any(same_expr(Reference(t.func, list(s.func.variables)), r) for r in known):
+            return False
+        return not all((plan.in_group(r.objectRef) and plan.stage_of(r.objectRef).inline) or
+                       any(same_expr(substitute_vars(r, ren), x) for x in known)
+                       for part in t.parts for r in plan._part_refs(part))
+
     def part_cond(s, pi, part, pnames, skip_box):
         conds = []
         if not skip_box:
@@ -581,7 +611,13 @@ def emit_group_kernel(pipe, plan, kname, threads, mode, xcd=True, forms=FORMS):
         for t in inline_closure(s):
             tn = ['q%d' % i for i in range(t.nd)]
             ww('%s v_%s = (%s)0;' % (c_type(t.func.typ), t.name, c_type(t.func.typ)), ind + 1)
-            ww('{', ind + 1)
+            if (s, t) not in needs:
+                needs[(s, t)] = conditional(s, t)
+            if needs[(s, t)]:
+                ww('if (%s) {' % ' && '.join('%s >= %s && %s <= %s' % (tn[i], R(t.region[i][0]), tn[i], R(t.region[i][1]))
+                                             for i in range(t.nd)), ind + 1)
+            else:
+                ww('{', ind + 1)
             ww('bool pmx_w = false;', ind + 2)
             emit_stage_value(out, t, 'v_' + t.name, tn, ind + 2, False, item)
             ww('(void)pmx_w;', ind + 2)
