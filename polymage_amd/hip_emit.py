@@ -1174,6 +1174,11 @@ def _forward_pair(plan, threads):
         if len(m1) != 1 or items(m1[0]) > threads:
             continue
         s1 = m1[0]
+        # (the first sweep keeps all its loads in registers, so all of them
+        # must happen at every point)
+        if any(len(t.parts) > 1 or t.parts[0].pred or t.parts[0].expr.has(Select)
+               for t in [s1] + [t for (t, r) in plan.closure_refs(s1)]):
+            continue
         for b in phs[a_i + 1:]:
             if len(by_phase[b]) != 1:
                 continue

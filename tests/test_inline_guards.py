@@ -1,6 +1,7 @@
 """General kernels with inlined stages that only a Case or a Select's branch
-reads, outside whose domain their reads leave the image or the tile's LDS:
-AddressSanitizer on the emulator, and the oracle's bits."""
+reads, outside whose domain their reads leave the image or the tile's LDS,
+and with a Case's loads that a later sweep reads again: AddressSanitizer on
+the emulator, and the oracle's bits."""
 import os
 import subprocess
 import sys
@@ -16,7 +17,7 @@ from polymage_amd.constructs import (Parameter, Variable, Interval, Image, Funct
 from helpers import build, bits_equal, gpu_build, emulating
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-FORMS = ['case', 'select', 'chain', 'rows']
+FORMS = ['case', 'select', 'chain', 'rows', 'forward']
 R_, C_ = 70, 100
 
 
@@ -39,16 +40,24 @@ def _check(form):
     elif form == 'chain':
         u = func('u', 30, t(x, y) * 0.5)
         out = func('out', 0, Select(here, u(x, y), img(x, y)))
+    elif form == 'forward':
+        a = func('a', 0, Case(here, img(x - 30, y) * 0.5 + img(x, y)), Case(Condition(x, '<', 30), img(x, y) * 2.0))
+        cols = Interval(Int, 1, C - 2)
+        two = a(x, y - 1) + a(x, y + 1) + img(x, y)
+        out = func('out', 0, Case(here, two + img(x - 30, y)), Case(Condition(x, '<', 30), two))
     else:
         # a stage in LDS of which a tile below row 30 computes nothing
         a = func('a', 30, img(x - 30, y) + img(x - 29, y))
         b = func('b', 31, a(x, y) + a(x - 1, y) * 0.5)
         out = func('out', 0, Case(Condition(x, '>=', 40), b(x, y)), Case(Condition(x, '<', 40), img(x, y)))
-    pipe = build(out, {'R': R, 'C': C}, {'R': 96, 'C': 128}, 'inlguard_' + form, [16, 16], gpu_options={'no_box': 1})
+    opts, tiles, c0 = {'no_box': 1}, [16, 16], C_
+    if form == 'forward':
+        opts, tiles, c0 = {'no_box': 1, 'threads': 128, 'block': (8, 1)}, [16, 60], C_ - 2
+    pipe = build(out, {'R': R, 'C': C}, {'R': 96, 'C': 128}, 'inlguard_' + form, tiles, gpu_options=opts)
     # (the oracle evaluates both branches of a Select: rows around the image)
     big = np.random.default_rng(4).random((R_ + 70, C_)).astype(np.float32)
     vals = {'R': R_, 'C': C_, 'img': big[35:35 + R_].copy()}
-    g = np.full((R_, C_), 7, np.float32)
+    g = np.full((R_, c0), 7, np.float32)
     o = g.copy()
     gpu_build(pipe).run_host(dict(vals, out=g))
     cemit.build([out], 'inlguard')(dict(vals, img=big[35:35 + R_], out=o))
